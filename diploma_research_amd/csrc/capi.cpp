@@ -45,6 +45,42 @@ void free_handle(dim_csr5* h) {
     delete h;
 }
 
+// The diagonal form of an uploaded format. A matrix without room for it does
+// without: its products then run the tile kernels.
+hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h) {
+    DiaForm D;
+    D.rows = f.rows;
+    D.cols = f.cols;
+    D.ld = (uint64_t{f.rows} + 63) / 64 * 64; // every diagonal starts on a 512-byte line
+    std::copy(f.dia_off.begin(), f.dia_off.end(), D.off);
+    const size_t n = size_t{f.dia_nd} * D.ld;
+    const size_t kept = h->allocations.size();
+    const uint64_t kept_bytes = h->device_bytes;
+    hipError_t e = upload(h, D.meta, f.dia_meta);
+    if (e == hipSuccess)
+        e = dev_alloc(h, D.v64, n);
+    if (e == hipSuccess && h->f.vals32)
+        e = dev_alloc(h, D.v32, n);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        for (; h->allocations.size() > kept; h->allocations.pop_back())
+            (void)hipFree(h->allocations.back());
+        h->device_bytes = kept_bytes;
+        return hipSuccess;
+    }
+    if (e == hipSuccess)
+        e = hipMemset(D.v64, 0, n * sizeof(double));
+    if (e == hipSuccess && D.v32)
+        e = hipMemset(D.v32, 0, n * sizeof(float));
+    if (e != hipSuccess)
+        return e;
+    D.nd = f.dia_nd;
+    D.products = f.dia_rows_in_two_lanes;
+    h->dia = D;
+    e = launch_dia_fill(h->f, D, nullptr);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+
 dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, bool plain_columns) {
     std::unique_ptr<dim_csr5, void (*)(dim_csr5*)> h(new dim_csr5, free_handle);
     DIM_HIP_TRY(hipGetDevice(&h->device));
@@ -110,6 +146,8 @@ dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, boo
     h->sys_tile = {0, f.tiles};
     h->sys_nnz_csr = {0, f.nnz};
     h->nnz_logical = f.nnz;
+    if (f.dia_nd && !plain_columns)
+        DIM_HIP_TRY(upload_diagonals(f, h.get()));
     *out = h.release();
     return DIM_SUCCESS;
 }
@@ -286,6 +324,8 @@ hipError_t plain_product(dim_csr5* h, bool f32, const void* x, void* y, hipStrea
             return e;
         return launch_slice_sum(f32, xs->ystack, xs->present, xs->present_rank, h->f.rows, h->xs_slices, y, st);
     }
+    if (h->dia.products)
+        return launch_dia_spmv(h->dia, f32, x, y, st);
     return launch_spmv(h->f, h->s, f32, 1, x, y, 0, h->f.tiles, 0, 0, h->f.n_empty, false, nullptr, st);
 }
 
@@ -642,6 +682,17 @@ dim_status dim_csr5_spmv_timed(const dim_csr5* A, dim_dtype dtype, const void* x
         if (e == hipSuccess)
             e = hipEventRecord(ev[2], st);
         fixup = true;
+    } else if (self->dia.products) {
+        // one kernel
+        const auto st = static_cast<hipStream_t>(stream);
+        e = hipEventRecord(ev[0], st);
+        if (e == hipSuccess)
+            e = launch_dia_spmv(self->dia, dtype == DIM_F32, x, y, st);
+        if (e == hipSuccess)
+            e = hipEventRecord(ev[1], st);
+        if (e == hipSuccess)
+            e = hipEventRecord(ev[2], st);
+        fixup = false;
     } else {
         e = launch_spmv_events(self->f, self->s, dtype == DIM_F32, x, y, ev[0], ev[1], ev[2],
                                static_cast<hipStream_t>(stream), &fixup);
@@ -727,6 +778,10 @@ dim_status dim_csr5_spmm(const dim_csr5* A, dim_dtype dtype, uint32_t k, const v
     auto* self = const_cast<dim_csr5*>(A);
     const auto st = static_cast<hipStream_t>(stream);
     const bool f32 = dtype == DIM_F32;
+    if (self->dia.products) {
+        DIM_HIP_TRY(launch_dia_spmm(self->dia, f32, static_cast<int>(k), X, Y, 0, 0, st));
+        return DIM_SUCCESS;
+    }
     if (k >= kRowMajorStagingK && A->f.rows && A->f.cols) {
         // From 6 sides on, the column-major product plus two transposes beats
         // gathering k-wide rows (one cache line per lane and side).
@@ -773,6 +828,11 @@ dim_status dim_csr5_spmm_colmajor(const dim_csr5* A, dim_dtype dtype, uint32_t k
     if (ldx < std::max<uint64_t>(A->f.cols, 1) || ldy < std::max<uint64_t>(A->f.rows, 1))
         return fail(DIM_INVALID_ARGUMENT, "leading dimension smaller than the column length");
     auto* self = const_cast<dim_csr5*>(A);
+    if (self->dia.products) {
+        DIM_HIP_TRY(launch_dia_spmm(self->dia, dtype == DIM_F32, static_cast<int>(k), X, Y, ldx, ldy,
+                                    static_cast<hipStream_t>(stream)));
+        return DIM_SUCCESS;
+    }
     DIM_HIP_TRY(launch_spmv(self->f, self->s, dtype == DIM_F32, static_cast<int>(k), X, Y, 0, A->f.tiles, 0, 0,
                             A->f.n_empty, false, nullptr, static_cast<hipStream_t>(stream), nullptr, ldx, ldy));
     return DIM_SUCCESS;
@@ -818,6 +878,8 @@ dim_status dim_csr5_set_values(dim_csr5* A, const double* vals, void* stream) {
         const DevFormat view = system_view(A, s);
         DIM_HIP_TRY(launch_set_values(view, vals + A->sys_nnz_csr[s], static_cast<hipStream_t>(stream)));
     }
+    if (A->dia.nd)
+        DIM_HIP_TRY(launch_dia_fill(A->f, A->dia, static_cast<hipStream_t>(stream)));
     return DIM_SUCCESS;
 }
 

@@ -59,6 +59,12 @@ struct HostFormat {
     // one of few diagonals and no row is empty.
     std::vector<int32_t> col_dict;  // the diagonals col - row, ascending
     std::vector<uint32_t> col_code; // T*64 words, see build_col_codes
+    // Diagonal form (see build_diagonals): dia_nd is 0 unless the matrix is
+    // kept by diagonals too.
+    uint32_t dia_nd = 0;
+    std::vector<int32_t> dia_off;   // dia_nd offsets col - row, ascending, then padding
+    std::vector<uint16_t> dia_meta; // one word per row
+    bool dia_rows_in_two_lanes = false; // no row spans three lanes
 };
 
 // Column codes: for matrices whose elements lie on few diagonals (col - row
@@ -72,7 +78,26 @@ constexpr uint32_t kMaxDiagonals = 16;
 constexpr uint32_t kMaxCodedSigma = 8;
 constexpr uint32_t kCodeFlagShift = 24;
 constexpr uint32_t code_bits(uint32_t sigma) { return sigma <= 6 ? 4 : 3; }
-void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx);
+void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx,
+                     const std::vector<int64_t>& diagonals);
+
+// Diagonal form: a matrix whose elements lie on at most kDiaMax diagonals,
+// nearly all of them full, is also kept by diagonals (v[d * ld + row]), so that
+// a product streams nothing but values and reads x in row order. Row i's word
+// in dia_meta says which diagonals it holds (bit d) and, above
+// kDiaSplitShift, at which diagonal the second lane's part of the row begins
+// (kDiaNoSplit: the row lies in one lane): the tile kernels add the part of a
+// row in one lane to its part in the next, and the diagonal form keeps that
+// order, so that both forms give the same bits. Rows must be no longer than
+// sigma (two lanes at most) for that; longer rows get kDiaNoSplit.
+// A missing element counts as padding: at most a quarter of the elements.
+constexpr uint32_t kDiaMax = 9;
+constexpr uint32_t kDiaSplitShift = 12;
+constexpr uint32_t kDiaNoSplit = 15;
+// diagonals with a compiled kernel: the smallest of 3, 5, 7, 9 that holds n
+constexpr uint32_t dia_kernel_diagonals(uint32_t n) { return n <= 3 ? 3 : n <= 5 ? 5 : n <= 7 ? 7 : 9; }
+void build_diagonals(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx,
+                     const std::vector<int64_t>& diagonals);
 
 // Builds the format from CSR. Returns an empty string or an error message.
 std::string build_format(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t* row_ptr,

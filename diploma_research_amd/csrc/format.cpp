@@ -10,6 +10,7 @@
 #include "dim_internal.h"
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <mutex>
 #include <thread>
@@ -40,6 +41,40 @@ void parallel_for(uint64_t n, F&& f) {
     }
     for (auto& t : th)
         t.join();
+}
+
+// The diagonals col - row of a matrix without empty rows, ascending; empty
+// when there are more than kMaxDiagonals, one lies beyond 32 bits, or x is
+// not below 4 GB (products of matrices kept by diagonals address x with
+// 32-bit byte offsets). Gathered per thread range and merged.
+std::vector<int64_t> find_diagonals(const HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx) {
+    if (f.any_dirty || !f.nnz || !f.empty_rows.empty() || uint64_t{f.cols} * sizeof(double) > (uint64_t{1} << 32))
+        return {};
+    std::vector<int64_t> all;
+    std::mutex m;
+    bool too_many = false;
+    parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
+        std::vector<int64_t> d;
+        for (uint64_t r = b; r < e && d.size() <= kMaxDiagonals; ++r)
+            for (uint32_t k = row_ptr[r]; k < row_ptr[r + 1]; ++k) {
+                const int64_t v = int64_t{col_idx[k]} - static_cast<int64_t>(r);
+                if (std::find(d.begin(), d.end(), v) == d.end()) {
+                    d.push_back(v);
+                    if (d.size() > kMaxDiagonals)
+                        break;
+                }
+            }
+        std::lock_guard<std::mutex> g(m);
+        if (d.size() > kMaxDiagonals)
+            too_many = true;
+        else
+            all.insert(all.end(), d.begin(), d.end());
+    });
+    std::sort(all.begin(), all.end());
+    all.erase(std::unique(all.begin(), all.end()), all.end());
+    if (too_many || all.size() > kMaxDiagonals || all.front() < INT32_MIN || all.back() > INT32_MAX)
+        return {};
+    return all;
 }
 
 } // namespace
@@ -188,47 +223,20 @@ std::string build_format(uint32_t rows, uint32_t cols, uint64_t nnz, const uint3
     for (uint64_t r = 0; r < rows; ++r)
         if (row_ptr[r] == row_ptr[r + 1])
             f.empty_rows.push_back(static_cast<uint32_t>(r));
-    build_col_codes(f, row_ptr, col_idx);
+    const std::vector<int64_t> diagonals = find_diagonals(f, row_ptr, col_idx);
+    build_col_codes(f, row_ptr, col_idx, diagonals);
+    build_diagonals(f, row_ptr, col_idx, diagonals);
     return {};
 }
 
-void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx) {
+void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx,
+                     const std::vector<int64_t>& all) {
     f.col_dict.clear();
     f.col_code.clear();
-    // (products of coded matrices address x with 32-bit byte offsets)
-    if (f.sigma > kMaxCodedSigma || f.any_dirty || !f.nnz || !f.empty_rows.empty() ||
-        uint64_t{f.cols} * sizeof(double) > (uint64_t{1} << 32))
+    if (f.sigma > kMaxCodedSigma || all.empty())
         return;
-    // the diagonals, gathered per thread range and merged; more than
-    // kMaxDiagonals (or one beyond 32-bit range) means no codes
-    std::vector<std::vector<int64_t>> parts;
-    std::mutex m;
-    bool too_many = false;
-    parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
-        std::vector<int64_t> d;
-        for (uint64_t r = b; r < e && d.size() <= kMaxDiagonals; ++r)
-            for (uint32_t k = row_ptr[r]; k < row_ptr[r + 1]; ++k) {
-                const int64_t v = int64_t{col_idx[k]} - static_cast<int64_t>(r);
-                if (std::find(d.begin(), d.end(), v) == d.end()) {
-                    d.push_back(v);
-                    if (d.size() > kMaxDiagonals)
-                        break;
-                }
-            }
-        std::lock_guard<std::mutex> g(m);
-        if (d.size() > kMaxDiagonals)
-            too_many = true;
-        parts.push_back(std::move(d));
-    });
-    if (too_many)
-        return;
-    std::vector<int64_t> all;
-    for (auto& d : parts)
-        all.insert(all.end(), d.begin(), d.end());
-    std::sort(all.begin(), all.end());
-    all.erase(std::unique(all.begin(), all.end()), all.end());
     const uint32_t cb = code_bits(f.sigma);
-    if (all.size() > (1u << cb) || all.front() < INT32_MIN || all.back() > INT32_MAX)
+    if (all.size() > (1u << cb))
         return;
     f.col_dict.assign(all.begin(), all.end());
     // code of every element (padding: code 0), packed per tile column with
@@ -252,6 +260,51 @@ void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col
             f.col_code[w] = word;
         }
     });
+}
+
+void build_diagonals(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx,
+                     const std::vector<int64_t>& all) {
+    f.dia_nd = 0;
+    f.dia_off.clear();
+    f.dia_meta.clear();
+    f.dia_rows_in_two_lanes = false;
+    // (rows plus an offset stay within 32 bits)
+    if (all.empty() || all.size() > kDiaMax || f.rows > (1u << 30))
+        return;
+    const uint32_t nd = dia_kernel_diagonals(static_cast<uint32_t>(all.size()));
+    if (uint64_t{nd} * f.rows * 4 > f.nnz * 5)
+        return;
+    f.dia_meta.resize(f.rows);
+    std::atomic<bool> ordered{true};
+    parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
+        for (uint64_t r = b; r < e; ++r) {
+            const uint32_t e0 = row_ptr[r], len = row_ptr[r + 1] - e0;
+            const uint32_t left = f.sigma - e0 % f.sigma; // elements up to the lane's end
+            uint32_t held = 0, split = kDiaNoSplit, d = 0;
+            for (uint32_t k = 0; k < len; ++k) {
+                const int64_t v = int64_t{col_idx[e0 + k]} - static_cast<int64_t>(r);
+                while (d < all.size() && all[d] != v)
+                    ++d;
+                if (d == all.size()) { // columns out of order, or one twice
+                    ordered.store(false, std::memory_order_relaxed);
+                    return;
+                }
+                held |= 1u << d;
+                if (k == left && len <= f.sigma)
+                    split = d;
+                ++d;
+            }
+            f.dia_meta[r] = static_cast<uint16_t>(held | split << kDiaSplitShift);
+        }
+    });
+    if (!ordered.load()) {
+        f.dia_meta.clear();
+        return;
+    }
+    f.dia_nd = nd;
+    f.dia_rows_in_two_lanes = all.size() <= f.sigma;
+    f.dia_off.assign(all.begin(), all.end());
+    f.dia_off.resize(kDiaMax, 0);
 }
 
 } // namespace dimgpu

@@ -2,6 +2,7 @@
 // C ABI translation units.
 #pragma once
 
+#include "dia.h"
 #include "dim_internal.h"
 #include "kernels.h"
 #include "../../include/dim_gpu.h"
@@ -35,6 +36,7 @@ struct dim_csr5 {
     uint32_t* d_sys_chunk = nullptr;
     uint64_t nnz_logical = 0; // stored elements (the format's nnz counts padding inside a batch)
     dimgpu::BoundaryInfo binfo; // host copy of the tile flags (f.binfo points here)
+    dimgpu::DiaForm dia;        // stencil matrices: the values by diagonal (dia.h)
     // Column slices for plain products (capi.cpp): xs is the matrix whose
     // rows are the (column slice s, row i) pairs that hold elements, in the
     // order of s*rows + i. That stacked handle also owns the partial products

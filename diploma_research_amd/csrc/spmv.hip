@@ -39,14 +39,6 @@ __global__ void k_fill(V* y, size_t n, V value, const int* done) {
         y[i] = value;
 }
 
-// Row of the element at step r of this lane, from the lane's bit flags.
-__device__ __forceinline__ uint32_t element_row(uint32_t bits, int r, int y_off, uint32_t row0, bool dirty,
-                                                const uint32_t* tdo) {
-    const uint32_t upto = (r >= 31) ? 0xFFFFFFFFu : ((2u << r) - 1u);
-    const int s = y_off - 1 + __popc(bits & upto);
-    return row0 + (dirty ? tdo[s] : static_cast<uint32_t>(s));
-}
-
 // y[col] += a_ij * x[row] for every element: the transposed product scatters
 // into y with hardware floating-point atomics.
 template<typename V, int SIGMA>

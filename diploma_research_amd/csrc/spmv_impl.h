@@ -173,6 +173,14 @@ __device__ __forceinline__ uint32_t sload_flag(const uint8_t* p) {
     return (w >> ((a & 3u) * 8u)) & 0xffu;
 }
 
+// Row of the element at step r of this lane, from the lane's bit flags.
+__device__ __forceinline__ uint32_t element_row(uint32_t bits, int r, int y_off, uint32_t row0, bool dirty,
+                                                const uint32_t* tdo) {
+    const uint32_t upto = (r >= 31) ? 0xFFFFFFFFu : ((2u << r) - 1u);
+    const int s = y_off - 1 + __popc(bits & upto);
+    return row0 + (dirty ? tdo[s] : static_cast<uint32_t>(s));
+}
+
 // per-chunk flags written by the tile kernel
 constexpr uint8_t kChunkStarts = 1; // the chunk's first element starts a row
 constexpr uint8_t kChunkHead = 2;   // head slot holds the closing part of a row from earlier chunks
