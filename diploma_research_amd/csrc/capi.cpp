@@ -1,6 +1,7 @@
 // C ABI of libdim_gpu.so: matrix construction, products and the autotuner.
 // The CG entry points live in cg.hip.
 #include "handle.h"
+#include "resident.h"
 
 #include <hip/hip_runtime.h>
 
@@ -47,7 +48,7 @@ void free_handle(dim_csr5* h) {
 
 // The diagonal form of an uploaded format. A matrix without room for it does
 // without: its products then run the tile kernels.
-hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h) {
+hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h, bool products) {
     DiaForm D;
     D.rows = f.rows;
     D.cols = f.cols;
@@ -75,7 +76,7 @@ hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h) {
     if (e != hipSuccess)
         return e;
     D.nd = f.dia_nd;
-    D.products = f.dia_rows_in_two_lanes;
+    D.products = products && f.dia_rows_in_two_lanes;
     h->dia = D;
     e = launch_dia_fill(h->f, D, nullptr);
     return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
@@ -146,8 +147,10 @@ dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, boo
     h->sys_tile = {0, f.tiles};
     h->sys_nnz_csr = {0, f.nnz};
     h->nnz_logical = f.nnz;
-    if (f.dia_nd && !plain_columns)
-        DIM_HIP_TRY(upload_diagonals(f, h.get()));
+    // (with 32-bit columns only for the solver, whose iterates do not depend on
+    // the columns' form)
+    if (f.dia_nd && (!plain_columns || (f.rows == f.cols && f.rows <= kResidentRows)))
+        DIM_HIP_TRY(upload_diagonals(f, h.get(), !plain_columns));
     *out = h.release();
     return DIM_SUCCESS;
 }

@@ -5,6 +5,8 @@
 // 102-127): As = A*s; alpha = r.r / s.As; x += alpha*s; r -= alpha*As;
 // r.r_new; stop test; beta = r.r_new / r.r; s = r + beta*s.
 //
+// Systems of matrices kept by diagonals that fit the chip's registers and LDS
+// iterate in one launch of resident workgroups (resident.hip); the rest here.
 // One iteration is four kernels with every scalar kept on the device:
 //   1. CSR5 tiles  q = A p, with p[row]*q[row] folded into the epilogue;
 //   2. carry fix-up of rows that cross tiles, which also reduces the p.q
@@ -24,6 +26,7 @@
 // batches: x += x_corr, r = b - A x, both in FP64, and the stop test uses that
 // FP64 residual (reliable updates).
 #include "handle.h"
+#include "resident.h"
 
 #include <hip/hip_runtime.h>
 
@@ -61,6 +64,9 @@ struct CgState {
     // block (0, 0) sets `done` at its end, and a block of the same launch
     // that starts after that must still apply this iteration's x update.
     int done_prev;
+    // the resident solver's columns stop one by one
+    int col_run[kMaxK];   // iterations of the column so far
+    double pause[kMaxK];  // FP32-refined: r.r below which its residual is replaced
 };
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -156,7 +162,7 @@ __global__ __launch_bounds__(kVecThreads) void k_cg_init(size_t n, const double*
 // Tolerances and the initial stop test (one block).
 template<int KMAX>
 __global__ void k_cg_init_state(CgState* st, int nparts, const double* rr_part, const double* bb_part, double rtol,
-                                double* hist) {
+                                double delta2, double* hist) {
     __shared__ double rr[KMAX], bb[KMAX];
     const int k = st->k;
     reduce_parts<KMAX>(rr_part, nparts, k, rr);
@@ -172,6 +178,8 @@ __global__ void k_cg_init_state(CgState* st, int nparts, const double* rr_part, 
             st->rr_true[j] = rr[j];
             st->col_done[j] = rr[j] <= st->tol2[j] ? 1 : 0;
             st->col_iters[j] = 0;
+            st->col_run[j] = 0;
+            st->pause[j] = delta2 * rr[j];
             all &= st->col_done[j] != 0;
             if (hist)
                 hist[j] = std::sqrt(rr[j]) / scale;
@@ -320,28 +328,36 @@ __global__ __launch_bounds__(kVecThreads) void k_ru_residual(const CgState* st, 
 }
 
 // Reliable update, part 3 (one block): the FP64 stop test decides; columns
-// whose FP64 residual is not yet small enough are resumed.
+// whose FP64 residual is not yet small enough are resumed. own_count: every
+// column has its own iteration count (the resident solver), else they share
+// the state's.
 template<int KMAX>
-__global__ void k_ru_state(CgState* st, int nparts, const double* rr_part, const double* rt_part) {
+__global__ void k_ru_state(CgState* st, int nparts, const double* rr_part, const double* rt_part, double delta2,
+                           bool own_count) {
     __shared__ double rr[KMAX], rt[KMAX];
     const int k = st->k;
     reduce_parts<KMAX>(rr_part, nparts, k, rr);
     reduce_parts<KMAX>(rt_part, nparts, k, rt);
     if (threadIdx.x == 0) {
-        int all = 1;
+        int all = 1, more = 0;
         for (int j = 0; j < k; ++j) {
+            const int it = own_count ? st->col_run[j] : st->iterations;
             st->rr[j] = rr[j];
             st->rr_true[j] = rt[j];
+            st->pause[j] = delta2 * rr[j];
             if (st->col_done[j] != 2) {
                 const int c = rt[j] <= st->tol2[j];
                 if (c && st->col_done[j] != 1)
-                    st->col_iters[j] = st->iterations;
+                    st->col_iters[j] = it;
                 st->col_done[j] = c;
+            } else if (own_count) {
+                st->done = 2;
             }
             all &= st->col_done[j] != 0;
+            more |= !st->col_done[j] && it < st->max_iters;
         }
         if (st->done != 2)
-            st->done = all ? 1 : (st->iterations >= st->max_iters ? 3 : 0);
+            st->done = all ? 1 : (more ? 0 : 3);
     }
 }
 
@@ -442,6 +458,28 @@ struct Launcher {
     }
 };
 
+// Y = A X in FP64 on n x k column-major blocks.
+hipError_t plain_product(dim_csr5* A, int k, const double* x, double* y, size_t n, hipStream_t s) {
+    if (A->dia.products)
+        return k == 1 ? launch_dia_spmv(A->dia, false, x, y, s) : launch_dia_spmm(A->dia, false, k, x, y, n, n, s);
+    return launch_spmv(A->f, A->s, false, k, x, y, 0, A->f.tiles, 0, 0, A->f.n_empty, false, nullptr, s, nullptr, n);
+}
+
+// The resident solver's plan for k right-hand sides of a matrix kept by
+// diagonals: one job per column of the column-major blocks.
+ResidentPlan resident_plan(const dim_csr5* A, int k, bool mixed) {
+    if (!A->dia.nd || (mixed && !A->dia.v32))
+        return {};
+    std::vector<ResidentJob> jobs(static_cast<size_t>(k));
+    for (int j = 0; j < k; ++j) {
+        jobs[j].row0 = 0;
+        jobs[j].rows = A->f.rows;
+        jobs[j].vec0 = static_cast<uint64_t>(j) * A->f.rows;
+        std::copy(std::begin(A->dia.off), std::end(A->dia.off), jobs[j].off);
+    }
+    return plan_resident(std::move(jobs), A->dia.nd, mixed ? sizeof(float) : sizeof(double));
+}
+
 // The device buffers of one solve: the state, the reduction partials (nvb *
 // kMaxK each), the work vectors of the precision in use and, for k > 1, the
 // column-major copies of B and X.
@@ -450,9 +488,15 @@ struct Work {
     double *rr0 = nullptr, *rr1 = nullptr, *bb = nullptr, *rt = nullptr, *hist = nullptr;
     double *q64 = nullptr, *r64 = nullptr, *p64 = nullptr, *bc = nullptr, *xc = nullptr;
     float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *x32 = nullptr;
+    char* res = nullptr; // the resident solver's workspace, of res_bytes bytes
+    size_t res_bytes = 0;
 };
 
-dim_status alloc_work(DevBuf& buf, size_t n, int k, uint32_t nvb, bool mixed, int hist_cap, Work& w) {
+dim_status alloc_work(DevBuf& buf, size_t n, int k, uint32_t nvb, bool mixed, int hist_cap, size_t res_bytes, Work& w) {
+    if (res_bytes) {
+        DIM_HIP_TRY(buf.alloc(w.res, res_bytes));
+        w.res_bytes = res_bytes;
+    }
     DIM_HIP_TRY(buf.alloc(w.st, 1));
     DIM_HIP_TRY(buf.alloc(w.q64, n * k));
     DIM_HIP_TRY(buf.alloc(w.rr0, size_t{nvb} * kMaxK));
@@ -501,6 +545,8 @@ struct CgCache {
     int k = 0;
     bool mixed = false;
     int hist_cap = 0;
+    ResidentPlan plan;
+    bool plan_uploaded = false;
     PinnedState pinned;
     hipStream_t cap = nullptr;
     Graph graph;
@@ -537,7 +583,9 @@ dim_status cg_cache_for(dim_csr5* A, size_t n, int k, uint32_t nvb, bool mixed, 
     free_cg_cache(c);
     A->cg_cache = nullptr;
     std::unique_ptr<CgCache> fresh(new CgCache);
-    if (dim_status e = alloc_work(fresh->buf, n, k, nvb, mixed, hist_cap, fresh->w))
+    fresh->plan = resident_plan(A, k, mixed);
+    if (dim_status e = alloc_work(fresh->buf, n, k, nvb, mixed, hist_cap,
+                                  fresh->plan.ok ? resident_bytes(fresh->plan) : 0, fresh->w))
         return e;
     DIM_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&fresh->pinned.h), sizeof(CgState), hipHostMallocDefault));
     DIM_HIP_TRY(hipStreamCreateWithFlags(&fresh->cap, hipStreamNonBlocking));
@@ -572,16 +620,25 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
     DevBuf buf;
     Work w;
     CgCache* cc = nullptr; // the handle's buffers, when this solve's fit them
+    ResidentPlan own_plan;
     if (no_alloc) {
         w = *fixed;
+        own_plan = resident_plan(A, k, mixed);
     } else {
         if (dim_status e = cg_cache_for(A, n, k, nvb, mixed, hist_cap, &cc))
             return e;
-        if (cc)
+        if (cc) {
             w = cc->w;
-        else if (dim_status e = alloc_work(buf, n, k, nvb, mixed, hist_cap, w))
-            return e;
+        } else {
+            own_plan = resident_plan(A, k, mixed);
+            if (dim_status e = alloc_work(buf, n, k, nvb, mixed, hist_cap,
+                                          own_plan.ok ? resident_bytes(own_plan) : 0, w))
+                return e;
+        }
     }
+    const ResidentPlan& plan = cc ? cc->plan : own_plan;
+    bool resident = plan.ok && resident_bytes(plan) <= w.res_bytes;
+    bool upload_plan = !(cc && cc->plan_uploaded);
     CgState* st = w.st;
     double *q64 = w.q64, *r64 = w.r64, *p64 = w.p64, *rr0 = w.rr0, *rr1 = w.rr1, *bb = w.bb, *rt = w.rt,
            *hist = w.hist;
@@ -617,35 +674,40 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
     // of the same iterations
     Graph graph;
     hipGraphExec_t exec = nullptr;
-    if (cc && cc->graph.ge && cc->g_kmax == KMAX && cc->g_check == check && cc->g_x == x) {
-        exec = cc->graph.ge;
-    } else if (!no_alloc) {
-        Graph& gr = cc ? cc->graph : graph;
-        gr.reset();
-        hipStream_t cap = cc ? cc->cap : nullptr;
-        if (!cc)
-            DIM_HIP_TRY(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-        bool ok = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal) == hipSuccess;
-        if (ok) {
-            enqueue_batch(cap);
-            ok = hipStreamEndCapture(cap, &gr.g) == hipSuccess && gr.g &&
-                 hipGraphInstantiate(&gr.ge, gr.g, nullptr, nullptr, 0) == hipSuccess;
-            (void)hipGetLastError();
-        }
-        if (!cc)
-            (void)hipStreamDestroy(cap);
-        if (ok) {
-            exec = gr.ge;
-            if (cc) {
-                cc->g_kmax = KMAX;
-                cc->g_check = check;
-                cc->g_x = x;
-            }
-        } else {
+    auto capture = [&]() -> dim_status {
+        if (cc && cc->graph.ge && cc->g_kmax == KMAX && cc->g_check == check && cc->g_x == x) {
+            exec = cc->graph.ge;
+        } else if (!no_alloc) {
+            Graph& gr = cc ? cc->graph : graph;
             gr.reset();
+            hipStream_t cap = cc ? cc->cap : nullptr;
+            if (!cc)
+                DIM_HIP_TRY(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
+            bool ok = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal) == hipSuccess;
+            if (ok) {
+                enqueue_batch(cap);
+                ok = hipStreamEndCapture(cap, &gr.g) == hipSuccess && gr.g &&
+                     hipGraphInstantiate(&gr.ge, gr.g, nullptr, nullptr, 0) == hipSuccess;
+                (void)hipGetLastError();
+            }
+            if (!cc)
+                (void)hipStreamDestroy(cap);
+            if (ok) {
+                exec = gr.ge;
+                if (cc) {
+                    cc->g_kmax = KMAX;
+                    cc->g_check = check;
+                    cc->g_x = x;
+                }
+            } else {
+                gr.reset();
+            }
         }
-    }
-    const bool use_graph = exec != nullptr;
+        return DIM_SUCCESS;
+    };
+    if (!resident)
+        if (dim_status e = capture())
+            return e;
 
     hipEvent_t e0 = nullptr, e1 = nullptr;
     const auto t_start = std::chrono::steady_clock::now();
@@ -669,8 +731,7 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
     init.k = k;
     DIM_HIP_TRY(hipMemcpyAsync(st, &init, sizeof(CgState), hipMemcpyHostToDevice, stream));
     // q = A x0 (FP64), r = b - q, p = r
-    DIM_HIP_TRY(launch_spmv(A->f, A->s, false, k, x, q64, 0, A->f.tiles, 0, 0, A->f.n_empty, false, nullptr, stream,
-                            nullptr, n));
+    DIM_HIP_TRY(plain_product(A, k, x, q64, n, stream));
     if (mixed) {
         hipLaunchKernelGGL((k_cg_init<float>), vgrid, dim3(kVecThreads), 0, stream, n, b, q64, r32, p32, rr0, bb);
         hipLaunchKernelGGL((k_zero<float>), dim3(nvb), dim3(kVecThreads), 0, stream, x32, n * k);
@@ -678,16 +739,64 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         hipLaunchKernelGGL((k_cg_init<double>), vgrid, dim3(kVecThreads), 0, stream, n, b, q64, r64, p64, rr0, bb);
     }
     hipLaunchKernelGGL((k_cg_init_state<KMAX>), dim3(1), dim3(64), 0, stream, st, static_cast<int>(nvb), rr0, bb,
-                       o.rtol, hist);
+                       o.rtol, delta * delta, hist);
     DIM_HIP_TRY(hipGetLastError());
+
+    // Every column's iterations on the resident solver, until it stops (or,
+    // FP32-refined, its residual is to be replaced). A launch whose workgroups
+    // are not seated as the plan assumes says so before it touches anything;
+    // the launch sequence then does the work.
+    auto iterate_resident = [&]() -> dim_status {
+        ResidentState rs;
+        rs.tol2 = st->tol2;
+        rs.bnorm = st->bnorm;
+        rs.pause = mixed ? st->pause : nullptr;
+        rs.rr = st->rr;
+        rs.done = st->col_done;
+        rs.iters = st->col_iters;
+        rs.run = st->col_run;
+        rs.max_iters = static_cast<int>(o.max_iters);
+        rs.hist = hist;
+        rs.hist_cap = hist_cap;
+        std::lock_guard<std::mutex> guard(resident_mutex()); // (the stream is idle here)
+        DIM_HIP_TRY(launch_resident(plan, mixed, mixed ? static_cast<const void*>(A->dia.v32) : A->dia.v64, A->dia.ld,
+                                    mixed ? static_cast<void*>(x32) : x, mixed ? static_cast<void*>(r32) : r64,
+                                    mixed ? static_cast<void*>(p32) : p64, rs, w.res, upload_plan, stream));
+        upload_plan = false;
+        if (cc)
+            cc->plan_uploaded = true;
+        int code = 0;
+        DIM_HIP_TRY(resident_abort(w.res, &code, stream));
+        DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
+        DIM_HIP_TRY(hipStreamSynchronize(stream));
+        if (code == kResidentSeats) {
+            resident = false;
+            return capture();
+        }
+        if (code)
+            return fail(DIM_HIP_ERROR, "CG: a wait between the resident solver's workgroups timed out");
+        hs->iterations = 0;
+        bool broke = false;
+        int all = 1;
+        for (int j = 0; j < k; ++j) {
+            hs->iterations = std::max(hs->iterations, hs->col_run[j]);
+            broke = broke || hs->col_done[j] == 2;
+            all &= hs->col_done[j] != 0;
+        }
+        // (done columns still go through the FP64 test when refining)
+        hs->done = broke ? 2 : all ? 1 : hs->iterations >= static_cast<int>(o.max_iters) ? 3 : 0;
+        return DIM_SUCCESS;
+    };
 
     uint32_t refinements = 0;
     std::array<double, kMaxK> rr_at_update{};
     bool first = true;
     dim_status status = DIM_SUCCESS;
     for (;;) {
-        DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
-        DIM_HIP_TRY(hipStreamSynchronize(stream));
+        if (!resident || first) {
+            DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
+            DIM_HIP_TRY(hipStreamSynchronize(stream));
+        }
         if (first) {
             for (int j = 0; j < k; ++j)
                 rr_at_update[j] = hs->rr_true[j];
@@ -697,18 +806,17 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
             // residual replacement when a column's FP32 residual fell by delta
             // since the last one, when the FP32 residual says converged, or at
             // the iteration cap
-            bool need = hs->done == 1 || hs->done == 3;
+            bool need = hs->done == 1 || hs->done == 3 || resident;
             for (int j = 0; j < k && !need; ++j)
                 need = !hs->col_done[j] && hs->rr[j] < delta * delta * rr_at_update[j];
             if (need && hs->iterations > 0) {
                 ++refinements;
                 hipLaunchKernelGGL(k_ru_fold, dim3(nvb), dim3(kVecThreads), 0, stream, n * k, x, x32);
-                DIM_HIP_TRY(launch_spmv(A->f, A->s, false, k, x, q64, 0, A->f.tiles, 0, 0, A->f.n_empty, false,
-                                        nullptr, stream, nullptr, n));
+                DIM_HIP_TRY(plain_product(A, k, x, q64, n, stream));
                 hipLaunchKernelGGL(k_ru_residual, vgrid, dim3(kVecThreads), 0, stream, static_cast<const CgState*>(st),
                                    n, b, static_cast<const double*>(q64), r32, p32, rr0, rt);
                 hipLaunchKernelGGL((k_ru_state<KMAX>), dim3(1), dim3(64), 0, stream, st, static_cast<int>(nvb), rr0,
-                                   rt);
+                                   rt, delta * delta, resident);
                 DIM_HIP_TRY(hipGetLastError());
                 DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
                 DIM_HIP_TRY(hipStreamSynchronize(stream));
@@ -718,7 +826,12 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         }
         if (hs->done)
             break;
-        if (use_graph) {
+        if (resident) {
+            if (dim_status e = iterate_resident())
+                return e;
+            if (resident && !mixed)
+                break;
+        } else if (exec) {
             DIM_HIP_TRY(hipGraphLaunch(exec, stream));
         } else {
             enqueue_batch(stream);
@@ -727,8 +840,7 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
     }
     // true residual ||b - A x|| in FP64, and the solution back in the
     // caller's row-major layout
-    DIM_HIP_TRY(launch_spmv(A->f, A->s, false, k, x, q64, 0, A->f.tiles, 0, 0, A->f.n_empty, false, nullptr, stream,
-                            nullptr, n));
+    DIM_HIP_TRY(plain_product(A, k, x, q64, n, stream));
     hipLaunchKernelGGL(k_resid_parts, vgrid, dim3(kVecThreads), 0, stream, n, b, static_cast<const double*>(q64), rt);
     if (k > 1)
         hipLaunchKernelGGL(k_cols_to_rows, dim3(tgrid), dim3(256), 0, stream, n, k,
@@ -764,7 +876,7 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         const double scale = S.bnorm[j] > 0.0 ? S.bnorm[j] : 1.0;
         dim_cg_result& R = res[j];
         R.converged = S.col_done[j] == 1;
-        R.iterations = static_cast<uint32_t>(S.col_done[j] ? S.col_iters[j] : S.iterations);
+        R.iterations = static_cast<uint32_t>(S.col_done[j] ? S.col_iters[j] : resident ? S.col_run[j] : S.iterations);
         R.relres = std::sqrt(mixed ? S.rr_true[j] : S.rr[j]) / scale;
         R.relres_true = std::sqrt(tr) / scale;
         R.refinements = refinements;
@@ -796,14 +908,17 @@ dim_status run(dim_csr5* A, int k, const double* b, double* x, const dim_cg_opts
 
 // ---- allocation-free solves (dim_cg_noalloc) -------------------------------
 // One right-hand side of at most kNoAllocMaxRows rows. Layout of the array:
-// the state, four partial arrays (rr0, rr1, bb, rt), then q64 and either r64,
-// p64 (FP64) or r32, p32, q32, x32 (FP32-refined): 24 bytes per row either
-// way, each piece starting on a 256-byte boundary.
+// the state, four partial arrays (rr0, rr1, bb, rt), the resident solver's
+// workspace, then q64 and either r64, p64 (FP64) or r32, p32, q32, x32
+// (FP32-refined): 24 bytes per row either way, each piece starting on a
+// 256-byte boundary.
 constexpr size_t kNoAllocMaxRows = DIM_CG_NOALLOC_MAX_ROWS;
 constexpr size_t kNoAllocAlign = 256;
 constexpr size_t kNoAllocStateBytes = 1024;
-constexpr size_t kNoAllocPartBytes = size_t{kMaxVecBlocks} * kMaxK * sizeof(double);
-constexpr size_t kNoAllocBytes = kNoAllocStateBytes + 4 * kNoAllocPartBytes + 24 * kNoAllocMaxRows + 8 * kNoAllocAlign;
+constexpr size_t kNoAllocPartBytes = size_t{kMaxVecBlocks} * sizeof(double);
+constexpr size_t kNoAllocResidentBytes = 4 * (kMaxK - 1) * kNoAllocPartBytes;
+constexpr size_t kNoAllocBytes = kNoAllocStateBytes + 4 * kNoAllocPartBytes + kNoAllocResidentBytes +
+                                 24 * kNoAllocMaxRows + 8 * kNoAllocAlign;
 static_assert(sizeof(CgState) <= kNoAllocStateBytes, "CgState must fit its slot");
 static_assert(kNoAllocBytes == DIM_CG_NOALLOC_BYTES, "the header states the array's size");
 
@@ -845,6 +960,9 @@ Work carve_noalloc(char* base, size_t n, bool mixed) {
         *pp = reinterpret_cast<double*>(base + at);
         at += kNoAllocPartBytes;
     }
+    w.res = base + at;
+    w.res_bytes = kNoAllocResidentBytes;
+    at += kNoAllocResidentBytes;
     w.q64 = reinterpret_cast<double*>(base + at);
     at += up(n * sizeof(double));
     if (mixed) {
