@@ -14,6 +14,10 @@
 // A batch of iterations is captured once in a hipGraph and replayed until
 // every system has stopped; the host looks at the state between batches.
 //
+// Batches whose systems are kept by diagonals and fit the chip iterate on
+// resident workgroups instead (resident.hip), with either flag; what follows
+// is for the rest.
+//
 // With DIM_CG_PERSISTENT the same three phases run inside one persistent
 // cooperative kernel that keeps the whole iteration loop on the device,
 // separated by grid barriers (see k_b_persistent); its iterates are bitwise
@@ -27,6 +31,7 @@
 // fixed order, so iterates are reproducible (apart from the transposed
 // product, which scatters with atomics).
 #include "handle.h"
+#include "resident.h"
 #include "spmv_impl.h"
 
 #include <hip/hip_runtime.h>
@@ -70,7 +75,7 @@ std::string build_batched(const std::vector<SystemCsr>& sys, uint32_t sigma, Hos
     sys_tile.assign(1, 0);
     sys_nnz.assign(1, 0);
     uint64_t rows = 0, tiles = 0, tdo_total = 0;
-    bool codes = true;
+    bool codes = true, dia = true;
     std::vector<int32_t> dicts;
     for (const SystemCsr& s : sys) {
         HostFormat f;
@@ -103,6 +108,12 @@ std::string build_batched(const std::vector<SystemCsr>& sys, uint32_t sigma, Hos
             d.resize(kMaxDiagonals, 0);
             dicts.insert(dicts.end(), d.begin(), d.end());
         }
+        // the diagonal form (for the resident solver) needs every system's
+        dia = dia && f.dia_nd;
+        if (dia) {
+            out.dia_nd = std::max(out.dia_nd, f.dia_nd);
+            out.dia_off.insert(out.dia_off.end(), f.dia_off.begin(), f.dia_off.end());
+        }
         rows += s.rows;
         tiles += f.tiles;
         if (rows >= kDirty || tiles >= kDirty)
@@ -116,6 +127,10 @@ std::string build_batched(const std::vector<SystemCsr>& sys, uint32_t sigma, Hos
     } else {
         out.col_code.clear();
         out.col_dict.clear();
+    }
+    if (!dia || uint64_t{rows} > (1u << 30)) {
+        out.dia_nd = 0;
+        out.dia_off.clear();
     }
     out.rows = out.cols = static_cast<uint32_t>(rows);
     out.tiles = static_cast<uint32_t>(tiles);
@@ -167,6 +182,7 @@ struct SysArrays {
     int* done_alt;
     double* rr_alt;
     int* broke;
+    int* run;        // resident solver: the system's iterations so far
 };
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -260,6 +276,7 @@ __global__ void k_b_init_state(BState* st, SysArrays sa, Tables tb, const double
             sa.rr[s] = rr;
             sa.sys_done[s] = rr <= sa.tol2[s] ? 1 : 0;
             sa.sys_iters[s] = 0;
+            sa.run[s] = 0;
             all &= sa.sys_done[s] != 0;
         }
         __syncthreads();
@@ -800,6 +817,18 @@ void build_chunk_table(const std::vector<uint32_t>& sys_tile, uint64_t waves, st
     chunk_tile.push_back(static_cast<uint32_t>(T));
 }
 
+// The resident solver's plan for a batch: one job per system.
+ResidentPlan resident_batch(const std::vector<uint32_t>& sys_row, const std::vector<int32_t>& sys_off, uint32_t nd) {
+    std::vector<ResidentJob> jobs(sys_row.size() - 1);
+    for (size_t s = 0; s < jobs.size(); ++s) {
+        jobs[s].row0 = sys_row[s];
+        jobs[s].rows = sys_row[s + 1] - sys_row[s];
+        jobs[s].vec0 = sys_row[s];
+        std::copy(sys_off.begin() + s * kDiaMax, sys_off.begin() + (s + 1) * kDiaMax, jobs[s].off);
+    }
+    return plan_resident(std::move(jobs), nd, sizeof(double));
+}
+
 dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32_t>& sys_row,
                           const std::vector<uint32_t>& sys_tile, const std::vector<uint64_t>& sys_nnz, dim_csr5** out) {
     // upload_format keeps one dictionary; a batch keeps one per system
@@ -808,6 +837,9 @@ dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32
     const bool codes = !dicts.empty() && !f.col_code.empty();
     if (codes)
         f.col_dict.assign(dicts.begin(), dicts.begin() + kMaxDiagonals);
+    // and it fills its diagonal form itself
+    const uint32_t dia_nd = f.dia_nd;
+    f.dia_nd = 0;
     dim_csr5* h = nullptr;
     if (dim_status st = upload_format(f, keep_f32, &h))
         return st;
@@ -821,6 +853,26 @@ dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32
         int32_t* d = nullptr;
         DIM_HIP_TRY(upload(h, d, dicts));
         h->f.col_dict = d;
+    }
+    {
+        std::vector<SystemTiles> tab(h->n_systems);
+        for (uint32_t s = 0; s < h->n_systems; ++s)
+            tab[s] = {sys_tile[s], sys_tile[s + 1], sys_nnz[s], sys_nnz[s + 1] - sys_nnz[s]};
+        DIM_HIP_TRY(upload(h, h->sys_tab, tab));
+    }
+    // (only where the resident solver takes the batch)
+    if (dia_nd && resident_batch(sys_row, f.dia_off, dia_nd).ok) {
+        DiaForm D;
+        DIM_HIP_TRY(alloc_diagonals(h, dia_nd, D));
+        if (D.nd) {
+            int32_t* off = nullptr;
+            DIM_HIP_TRY(upload(h, off, f.dia_off));
+            D.sys_off = off;
+            h->dia = D;
+            h->sys_off = f.dia_off;
+            DIM_HIP_TRY(launch_dia_fill(h, nullptr));
+            DIM_HIP_TRY(hipStreamSynchronize(nullptr));
+        }
     }
     // chunk table: about one chunk per resident wavefront of the product
     // with its dot epilogue
@@ -929,6 +981,9 @@ struct BatchCache {
     BState* st = nullptr;
     SysArrays sa{};
     double *q = nullptr, *r = nullptr, *p = nullptr, *rr = nullptr, *pq = nullptr, *bb = nullptr, *rt = nullptr;
+    ResidentPlan plan;
+    char* res = nullptr; // the resident solver's workspace
+    bool plan_uploaded = false;
     BState* hs = nullptr; // pinned
     hipStream_t cap = nullptr;
     hipGraph_t graph = nullptr;
@@ -992,6 +1047,12 @@ dim_status init_batch_cache(dim_csr5* A, BatchCache& c) {
     DIM_HIP_TRY(m.alloc(sa.done_alt, S));
     DIM_HIP_TRY(m.alloc(sa.rr_alt, S));
     DIM_HIP_TRY(m.alloc(sa.broke, S));
+    DIM_HIP_TRY(m.alloc(sa.run, S));
+    if (A->dia.nd) {
+        c.plan = resident_batch(A->sys_row, A->sys_off, A->dia.nd);
+        if (c.plan.ok)
+            DIM_HIP_TRY(m.alloc(c.res, resident_bytes(c.plan)));
+    }
     DIM_HIP_TRY(m.alloc(c.q, n));
     DIM_HIP_TRY(m.alloc(c.r, n));
     DIM_HIP_TRY(m.alloc(c.p, n));
@@ -1010,8 +1071,8 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
     const bool transpose = (o.flags & DIM_CG_TRANSPOSE) != 0;
     const bool codes = A->f.col_code != nullptr;
     const bool persistent = (o.flags & DIM_CG_PERSISTENT) != 0;
-    const int occ = persistent ? persistent_occupancy(A->f.sigma, codes) : 0;
-    if (persistent && occ < 1)
+    const int occ = persistent && !A->dia.nd ? persistent_occupancy(A->f.sigma, codes) : 1;
+    if (occ < 1)
         return fail(DIM_UNSUPPORTED, "batched CG: the persistent kernel cannot be resident for this format");
     const size_t n = A->f.rows;
     const uint32_t check = o.check_every ? o.check_every : 16;
@@ -1059,7 +1120,34 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
                        static_cast<const double*>(bb), o.rtol);
     DIM_HIP_TRY(hipGetLastError());
 
-    if (persistent) {
+    // Systems kept by diagonals iterate on resident workgroups, side by side;
+    // where those cannot be seated (nothing is touched then) as below.
+    bool iterated = false;
+    if (bc->plan.ok && !transpose) {
+        ResidentState rs;
+        rs.tol2 = sa.tol2;
+        rs.bnorm = sa.bnorm;
+        rs.rr = sa.rr;
+        rs.done = sa.sys_done;
+        rs.iters = sa.sys_iters;
+        rs.run = sa.run;
+        rs.max_iters = static_cast<int>(o.max_iters);
+        DIM_HIP_TRY(hipStreamSynchronize(stream));
+        std::lock_guard<std::mutex> guard(resident_mutex());
+        DIM_HIP_TRY(launch_resident(bc->plan, false, A->dia.v64, A->dia.ld, x, r, p, rs, bc->res, !bc->plan_uploaded,
+                                    stream));
+        bc->plan_uploaded = true;
+        int code = 0;
+        DIM_HIP_TRY(resident_abort(bc->res, &code, stream));
+        DIM_HIP_TRY(hipStreamSynchronize(stream));
+        if (code && code != kResidentSeats)
+            return fail(DIM_HIP_ERROR, "batched CG: a wait between the resident solver's workgroups timed out");
+        iterated = !code;
+        hs->iterations = static_cast<int>(o.max_iters); // of the systems that have not stopped
+    }
+    if (iterated) {
+        // (done)
+    } else if (persistent) {
         // one cooperative launch runs every iteration; its vector work items
         // are the launch sequence's blocks (same rows, same reduction order)
         double *rr_part = nullptr, *dot_chunk = nullptr;

@@ -46,20 +46,14 @@ void free_handle(dim_csr5* h) {
     delete h;
 }
 
-// The diagonal form of an uploaded format. A matrix without room for it does
-// without: its products then run the tile kernels.
-hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h, bool products) {
-    DiaForm D;
-    D.rows = f.rows;
-    D.cols = f.cols;
-    D.ld = (uint64_t{f.rows} + 63) / 64 * 64; // every diagonal starts on a 512-byte line
-    std::copy(f.dia_off.begin(), f.dia_off.end(), D.off);
-    const size_t n = size_t{f.dia_nd} * D.ld;
+hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, DiaForm& D) {
+    D.rows = h->f.rows;
+    D.cols = h->f.cols;
+    D.ld = (uint64_t{h->f.rows} + 63) / 64 * 64; // every diagonal starts on a 512-byte line
+    const size_t n = size_t{nd} * D.ld;
     const size_t kept = h->allocations.size();
     const uint64_t kept_bytes = h->device_bytes;
-    hipError_t e = upload(h, D.meta, f.dia_meta);
-    if (e == hipSuccess)
-        e = dev_alloc(h, D.v64, n);
+    hipError_t e = dev_alloc(h, D.v64, n);
     if (e == hipSuccess && h->f.vals32)
         e = dev_alloc(h, D.v32, n);
     if (e == hipErrorOutOfMemory) {
@@ -67,18 +61,30 @@ hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h, bool products) {
         for (; h->allocations.size() > kept; h->allocations.pop_back())
             (void)hipFree(h->allocations.back());
         h->device_bytes = kept_bytes;
+        D = DiaForm{};
         return hipSuccess;
     }
     if (e == hipSuccess)
         e = hipMemset(D.v64, 0, n * sizeof(double));
     if (e == hipSuccess && D.v32)
         e = hipMemset(D.v32, 0, n * sizeof(float));
-    if (e != hipSuccess)
+    D.nd = nd;
+    return e;
+}
+
+// The diagonal form of an uploaded format. A matrix without room for it does
+// without: its products then run the tile kernels.
+static hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h, bool products) {
+    DiaForm D;
+    hipError_t e = alloc_diagonals(h, f.dia_nd, D);
+    if (e == hipSuccess && D.nd)
+        e = upload(h, D.meta, f.dia_meta);
+    if (e != hipSuccess || !D.nd)
         return e;
-    D.nd = f.dia_nd;
+    std::copy(f.dia_off.begin(), f.dia_off.end(), D.off);
     D.products = products && f.dia_rows_in_two_lanes;
     h->dia = D;
-    e = launch_dia_fill(h->f, D, nullptr);
+    e = launch_dia_fill(h, nullptr);
     return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
 }
 
@@ -178,30 +184,6 @@ std::vector<uint32_t> sigma_candidates(uint32_t rows, uint64_t nnz) {
     std::sort(c.begin(), c.end());
     c.erase(std::unique(c.begin(), c.end()), c.end());
     return c;
-}
-
-DevFormat system_view(const dim_csr5* A, uint32_t s) {
-    DevFormat view = A->f;
-    const uint32_t t0 = A->sys_tile[s], t1 = A->sys_tile[s + 1];
-    const size_t tile = size_t{kOmega} * A->f.sigma;
-    view.tiles = t1 - t0;
-    view.tile_ptr = A->f.tile_ptr + t0;
-    view.bit_flag = static_cast<char*>(A->f.bit_flag) + size_t{t0} * kOmega * (A->f.sigma <= 16 ? 2 : 4);
-    view.tile_flags = A->f.tile_flags + t0;
-    view.binfo_base = A->f.binfo_base + t0;
-    view.tile_desc_offset_ptr = A->f.tile_desc_offset_ptr + t0;
-    view.col_idx = A->f.col_idx + t0 * tile;
-    view.vals64 = A->f.vals64 + t0 * tile;
-    view.vals32 = A->f.vals32 ? A->f.vals32 + t0 * tile : nullptr;
-    view.col_code = A->f.col_code ? A->f.col_code + size_t{t0} * kOmega : nullptr;
-    // a batch with column codes keeps one table of diagonals per system
-    view.col_dict = A->f.col_dict && A->n_systems > 1 ? A->f.col_dict + size_t{s} * kMaxDiagonals : A->f.col_dict;
-    view.chunk_tile = nullptr;
-    view.chunk_sys = nullptr;
-    view.n_chunk_tab = 0;
-    view.nnz = A->sys_nnz_csr[s + 1] - A->sys_nnz_csr[s];
-    view.padded = size_t{view.tiles} * tile;
-    return view;
 }
 
 namespace {
@@ -858,10 +840,7 @@ dim_status dim_csr5_sampled_outer(const dim_csr5* A, double scale, const double*
         return st;
     if ((A->f.rows && !u) || (A->f.cols && !v) || (A->f.nnz && !out))
         return fail(DIM_INVALID_ARGUMENT, "null vector");
-    for (uint32_t s = 0; s < A->n_systems; ++s) {
-        const DevFormat view = system_view(A, s);
-        DIM_HIP_TRY(launch_sampled_outer(view, scale, u, v, out + A->sys_nnz_csr[s], static_cast<hipStream_t>(stream)));
-    }
+    DIM_HIP_TRY(launch_sampled_outer(A, scale, u, v, out, static_cast<hipStream_t>(stream)));
     return DIM_SUCCESS;
 }
 
@@ -877,12 +856,7 @@ dim_status dim_csr5_set_values(dim_csr5* A, const double* vals, void* stream) {
     free_handle(A->xs);
     A->xs = nullptr;
     A->xs_slices = 0;
-    for (uint32_t s = 0; s < A->n_systems; ++s) {
-        const DevFormat view = system_view(A, s);
-        DIM_HIP_TRY(launch_set_values(view, vals + A->sys_nnz_csr[s], static_cast<hipStream_t>(stream)));
-    }
-    if (A->dia.nd)
-        DIM_HIP_TRY(launch_dia_fill(A->f, A->dia, static_cast<hipStream_t>(stream)));
+    DIM_HIP_TRY(launch_set_values(A, vals, static_cast<hipStream_t>(stream)));
     return DIM_SUCCESS;
 }
 

@@ -18,17 +18,16 @@ struct DiaForm {
     uint32_t rows = 0, cols = 0;
     uint64_t ld = 0;
     int32_t off[kDiaMax] = {};
+    // batches: each system's offsets (kDiaMax of them), off unused; a system's
+    // rows follow one another as in the batch's vectors
+    const int32_t* sys_off = nullptr;
     double* v64 = nullptr;
     float* v32 = nullptr;
-    uint16_t* meta = nullptr;
+    uint16_t* meta = nullptr; // (not kept for batches)
     // plain products use it: the matrix keeps column codes or could, and no
     // row spans three lanes (the summation order is then the tile kernels')
     bool products = false;
 };
-
-// Writes the values of the diagonal form from the tile layout of A. The
-// places without an element are not written: they must hold 0.
-hipError_t launch_dia_fill(const DevFormat& A, const DiaForm& D, hipStream_t stream);
 
 // y = A x.
 hipError_t launch_dia_spmv(const DiaForm& D, bool f32, const void* x, void* y, hipStream_t stream);

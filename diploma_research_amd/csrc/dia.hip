@@ -13,9 +13,6 @@ namespace dimgpu {
 
 namespace {
 
-using detail::DescWord;
-using detail::element_row;
-using detail::wave_incl_scan;
 using detail::xcd_remap;
 
 struct DiaArgs {
@@ -157,40 +154,6 @@ __global__ __launch_bounds__(256) void k_dia_spmm_rows(DiaArgs a, uint32_t k, ui
         *reinterpret_cast<VW*>(Y + b0 * k + i * k + c) = s;
 }
 
-// Values of the diagonal form from the tile layout: one wavefront per tile,
-// every element's diagonal found among the nd offsets.
-template<int SIGMA>
-__global__ __launch_bounds__(256) void k_dia_fill(DevFormat A, DiaForm D) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= A.tiles)
-        return;
-    using W = typename DescWord<SIGMA>::type;
-    const size_t base = static_cast<size_t>(t) * (64 * SIGMA);
-    const uint32_t bits = static_cast<uint32_t>(static_cast<const W*>(A.bit_flag)[static_cast<size_t>(t) * 64 + lane]) |
-                          (lane == 0 ? 1u : 0u);
-    const uint32_t row0 = A.tile_ptr[t] & ~kDirty; // a matrix kept by diagonals has no dirty tiles
-    const int nb = __popc(bits);
-    const int y_off = wave_incl_scan(nb, lane) - nb;
-#pragma unroll
-    for (int r = 0; r < SIGMA; ++r) {
-        const size_t pos = base + static_cast<size_t>(r) * 64 + lane;
-        if (base + static_cast<size_t>(lane) * SIGMA + r >= A.nnz)
-            continue;
-        const uint32_t row = element_row(bits, r, y_off, row0, false, nullptr);
-        const int32_t diff = static_cast<int32_t>(A.col_idx[pos]) - static_cast<int32_t>(row);
-        uint32_t d = D.nd;
-#pragma unroll
-        for (int q = kDiaMax - 1; q >= 0; --q) // the first match: padding offsets come last
-            d = (static_cast<uint32_t>(q) < D.nd && D.off[q] == diff) ? static_cast<uint32_t>(q) : d;
-        if (d < D.nd && row < D.rows) {
-            D.v64[d * D.ld + row] = A.vals64[pos];
-            if (D.v32)
-                D.v32[d * D.ld + row] = A.vals32[pos];
-        }
-    }
-}
-
 DiaArgs make_args(const DiaForm& D) {
     DiaArgs a;
     a.meta = D.meta;
@@ -284,20 +247,6 @@ hipError_t spmm(const DiaForm& D, int k, const void* X, void* Y, uint64_t ldx, u
 }
 
 } // namespace
-
-hipError_t launch_dia_fill(const DevFormat& A, const DiaForm& D, hipStream_t stream) {
-    if (!A.tiles)
-        return hipSuccess;
-    const uint32_t grid = (A.tiles + 3) / 4;
-    switch (A.sigma) {
-#define DIM_DIA_FILL(S)                                                                                               \
-    case S: hipLaunchKernelGGL((k_dia_fill<S>), dim3(grid), dim3(256), 0, stream, A, D); break;
-        DIM_FOR_EACH_SIGMA(DIM_DIA_FILL)
-#undef DIM_DIA_FILL
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
 
 hipError_t launch_dia_spmv(const DiaForm& D, bool f32, const void* x, void* y, hipStream_t stream) {
     return f32 ? spmv<float>(D, x, y, stream) : spmv<double>(D, x, y, stream);

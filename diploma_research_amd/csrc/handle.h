@@ -17,6 +17,12 @@ struct CgCache;
 void free_cg_cache(CgCache* c);
 struct BatchCache;
 void free_batch_cache(BatchCache* c);
+// A system of a batch: tiles [tile0, tile1) and nnz elements from element nnz0
+// of the CSR order on.
+struct SystemTiles {
+    uint32_t tile0, tile1;
+    uint64_t nnz0, nnz;
+};
 } // namespace dimgpu
 
 struct dim_csr5 {
@@ -34,6 +40,9 @@ struct dim_csr5 {
     // chunks of system s in the chunk table: [sys_chunk[s], sys_chunk[s + 1])
     std::vector<uint32_t> sys_chunk;
     uint32_t* d_sys_chunk = nullptr;
+    // batches: tiles and elements of each system, on the device (values.hip)
+    dimgpu::SystemTiles* sys_tab = nullptr;
+    std::vector<int32_t> sys_off; // batches kept by diagonals: dia.sys_off's entries
     uint64_t nnz_logical = 0; // stored elements (the format's nnz counts padding inside a batch)
     dimgpu::BoundaryInfo binfo; // host copy of the tile flags (f.binfo points here)
     dimgpu::DiaForm dia;        // stencil matrices: the values by diagonal (dia.h)
@@ -112,8 +121,22 @@ hipError_t upload(dim_csr5* h, T*& p, const std::vector<T>& v) {
 // plain_columns: leave out the column codes (products stream col_idx).
 dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, bool plain_columns = false);
 
-// One system's share of a batched matrix as a stand-alone format view.
-DevFormat system_view(const dim_csr5* A, uint32_t s);
 void free_handle(dim_csr5* h);
+
+// New values (CSR order) into the tile layout, FP64 and, if kept, FP32, and into
+// the diagonal form.
+hipError_t launch_set_values(const dim_csr5* h, const double* vals_csr, hipStream_t stream);
+
+// out[e] = scale * u[row(e)] * v[col(e)] for every stored element e, in CSR order.
+hipError_t launch_sampled_outer(const dim_csr5* h, double scale, const double* u, const double* v, double* out,
+                                hipStream_t stream);
+
+// Writes the values of the diagonal form from the tile layout. The places
+// without an element are not written: they must hold 0.
+hipError_t launch_dia_fill(const dim_csr5* h, hipStream_t stream);
+
+// Device memory of a diagonal form with nd diagonals (values zeroed, FP32 ones
+// if the handle keeps them); hipSuccess with D.nd == 0 when there is no room.
+hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, DiaForm& D);
 
 } // namespace dimgpu

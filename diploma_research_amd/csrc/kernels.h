@@ -128,11 +128,4 @@ hipError_t launch_slice_sum(bool f32, const void* ystack, const uint32_t* presen
 hipError_t launch_block_transpose(bool f32, bool to_cols, size_t n, int k, const void* src, void* dst,
                                   hipStream_t stream);
 
-// Scatters CSR-order values into the tile layout (FP64, and FP32 if kept).
-hipError_t launch_set_values(const DevFormat& A, const double* vals_csr, hipStream_t stream);
-
-// out[e] = scale * u[row(e)] * v[col(e)] for every stored element e, in CSR order.
-hipError_t launch_sampled_outer(const DevFormat& A, double scale, const double* u, const double* v, double* out,
-                                hipStream_t stream);
-
 } // namespace dimgpu

@@ -74,55 +74,6 @@ __global__ __launch_bounds__(256) void k_csr5_transpose(TileParams p) {
     }
 }
 
-// out[csr(e)] = scale * u[row(e)] * v[col(e)]
-template<int SIGMA>
-__global__ __launch_bounds__(256) void k_sampled_outer(TileParams p, double scale, const double* u, const double* v,
-                                                       double* out) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= p.tile_end)
-        return;
-    using W = typename DescWord<SIGMA>::type;
-    const size_t base = static_cast<size_t>(t) * (64 * SIGMA);
-    const uint32_t bits = static_cast<uint32_t>(static_cast<const W*>(p.bit_flag)[static_cast<size_t>(t) * 64 + lane]) |
-                          (lane == 0 ? 1u : 0u);
-    const uint32_t tpw = p.tile_ptr[t];
-    const bool dirty = (tpw & kDirty) != 0;
-    const uint32_t row0 = tpw & ~kDirty;
-    const uint32_t* tdo = dirty ? p.tdo + p.tdo_ptr[t] : nullptr;
-    const int nb = __popc(bits);
-    const int y_off = wave_incl_scan(nb, lane) - nb;
-#pragma unroll
-    for (int r = 0; r < SIGMA; ++r) {
-        const size_t pos = base + static_cast<size_t>(r) * 64 + lane;
-        const size_t csr = base + static_cast<size_t>(lane) * SIGMA + r;
-        if (csr >= p.nnz)
-            continue;
-        const uint32_t row = element_row(bits, r, y_off, row0, dirty, tdo);
-        out[csr] = scale * u[row] * v[p.col_idx[pos]];
-    }
-}
-
-// Tile-layout values from CSR-order values: the same permutation as the
-// conversion's transpose, run on the device.
-template<int SIGMA>
-__global__ __launch_bounds__(256) void k_set_values(TileParams p, const double* src, double* v64, float* v32) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= p.tile_end)
-        return;
-    const size_t base = static_cast<size_t>(t) * (64 * SIGMA);
-#pragma unroll
-    for (int r = 0; r < SIGMA; ++r) {
-        const size_t pos = base + static_cast<size_t>(r) * 64 + lane;
-        const size_t csr = base + static_cast<size_t>(lane) * SIGMA + r;
-        const double a = csr < p.nnz ? src[csr] : 0.0;
-        v64[pos] = a;
-        if (v32)
-            v32[pos] = static_cast<float>(a);
-    }
-}
-
 TileParams make_tile_params(const DevFormat& A, bool f32) {
     TileParams tp{};
     tp.tile_ptr = A.tile_ptr;
@@ -505,39 +456,6 @@ hipError_t launch_spmv_transpose(const DevFormat& A, bool f32, const void* x, vo
         }
 #undef DIM_T_F
 #undef DIM_T_D
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_set_values(const DevFormat& A, const double* vals_csr, hipStream_t stream) {
-    if (!A.tiles)
-        return hipSuccess;
-    TileParams tp = make_tile_params(A, false);
-    const uint32_t grid = (A.tiles + 3) / 4;
-    switch (A.sigma) {
-#define DIM_SV(S)                                                                                                     \
-    case S:                                                                                                           \
-        hipLaunchKernelGGL((k_set_values<S>), dim3(grid), dim3(256), 0, stream, tp, vals_csr, A.vals64, A.vals32);   \
-        break;
-        DIM_FOR_EACH_SIGMA(DIM_SV)
-#undef DIM_SV
-        default: break;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_sampled_outer(const DevFormat& A, double scale, const double* u, const double* v, double* out,
-                                hipStream_t stream) {
-    if (!A.tiles)
-        return hipSuccess;
-    TileParams tp = make_tile_params(A, false);
-    const uint32_t grid = (A.tiles + 3) / 4;
-    switch (A.sigma) {
-#define DIM_O(S)                                                                                                      \
-    case S: hipLaunchKernelGGL((k_sampled_outer<S>), dim3(grid), dim3(256), 0, stream, tp, scale, u, v, out); break;
-        DIM_FOR_EACH_SIGMA(DIM_O)
-#undef DIM_O
-        default: break;
     }
     return hipGetLastError();
 }

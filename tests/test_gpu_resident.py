@@ -71,3 +71,39 @@ def test_indefinite_matrix_breaks_down(cuda, precision):
     A = Csr5.from_csr((n, n, rp, ci, -v), sigma=8, keep_f32=True)
     with pytest.raises(DimError, match="breakdown"):
         conjugate_gradient(A, to_dev(b), precision=precision)
+
+
+@pytest.mark.parametrize("sides", [[9] * 7 + [33], [5, 8, 40, 13] * 75, [350, 300, 20, 3, 280, 64, 64, 90, 340, 12]],
+                         ids=["eight", "take turns", "uneven"])
+def test_batches(cuda, sides):
+    """A batch of a system per XCD, of more systems than an XCD has
+    workgroups, and of very uneven ones: every system's solution, the capped
+    iterate, and the persistent form's bits."""
+    import torch
+
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    systems = []
+    for i, s in enumerate(sides):
+        rp, ci, v = matgen.varcoef((max(3, s * 3 // 4), s), 0.5, seed=i)
+        systems.append((len(rp) - 1, rp, ci, v))
+    A = Csr5.from_csr_batched(systems, sigma=5)
+    rng = np.random.default_rng(len(sides))
+    bs = [rng.uniform(-1, 1, n) for n, *_ in systems]
+    b = to_dev(np.concatenate(bs))
+    X, res = conjugate_gradient_batched(A, b, rtol=1e-10, max_iters=5000)
+    Xp, resp = conjugate_gradient_batched(A, b, rtol=1e-10, max_iters=5000, persistent=True)
+    assert torch.equal(X, Xp) and [r.iterations for r in res] == [r.iterations for r in resp]
+    Xc, resc = conjugate_gradient_batched(A, b, rtol=1e-14, max_iters=6)
+    X, Xc = X.cpu().numpy(), Xc.cpu().numpy()
+    off = 0
+    for i, ((n, rp, ci, v), bb) in enumerate(zip(systems, bs)):
+        if i < 12:
+            M = O.Csr5(n, n, rp, ci, v)
+            oc = M.cg(bb, rtol=1e-10, maxit=5000, nthreads=8)
+            assert res[i].converged and res[i].relres_true <= 1.01e-10
+            np.testing.assert_allclose(X[off: off + n], oc["x"], rtol=1e-7, atol=1e-8)
+            oc = M.cg(bb, rtol=1e-14, maxit=6, nthreads=8)
+            assert not resc[i].converged and resc[i].iterations == 6
+            np.testing.assert_allclose(Xc[off: off + n], oc["x"], rtol=1e-9, atol=1e-11)
+        off += n
