@@ -893,12 +893,13 @@ dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32
 }
 
 // sys_done (may be null): chunks of stopped systems are skipped.
-hipError_t product(dim_csr5* A, bool transpose, const double* x, double* y, const int* done, hipStream_t s,
+dim_status product(dim_csr5* A, bool transpose, const double* x, double* y, const int* done, hipStream_t s,
                    const int* sys_done = nullptr) {
     if (transpose)
-        return launch_spmv_transpose(A->f, false, x, y, s, done);
-    return launch_spmv(A->f, A->s, false, 1, x, y, 0, A->f.tiles, 0, 0, A->f.n_empty, false, done, s, nullptr, 0, 0,
-                       nullptr, sys_done);
+        return launch_spmv_transpose(A, false, x, y, s, done);
+    DIM_HIP_TRY(launch_spmv(A->f, A->s, false, 1, x, y, 0, A->f.tiles, 0, 0, A->f.n_empty, false, done, s, nullptr, 0, 0,
+                            nullptr, sys_done));
+    return DIM_SUCCESS;
 }
 
 // Vector work items: blocks of at most `rows_per` rows of one system.
@@ -925,7 +926,8 @@ dim_status report(dim_csr5* A, const double* b, double* x, bool transpose, const
                   uint32_t threads, const BState& hs, float ms, dim_cg_result* res, hipStream_t stream) {
     const uint32_t S = A->n_systems;
     // FP64 true residual of every system
-    DIM_HIP_TRY(product(A, transpose, x, q, nullptr, stream));
+    if (dim_status e = product(A, transpose, x, q, nullptr, stream))
+        return e;
     (void)threads;
     hipLaunchKernelGGL(k_b_resid, dim3(B), dim3(kThreads), 0, stream, tb, b, static_cast<const double*>(q), rt);
     DIM_HIP_TRY(hipGetLastError());
@@ -1113,7 +1115,8 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
     DIM_HIP_TRY(hipEventRecord(e0, stream));
     BState init{0, 0, static_cast<int>(o.max_iters), static_cast<int>(S), 0};
     DIM_HIP_TRY(hipMemcpyAsync(st, &init, sizeof(BState), hipMemcpyHostToDevice, stream));
-    DIM_HIP_TRY(product(A, transpose, x, q, nullptr, stream));
+    if (dim_status e = product(A, transpose, x, q, nullptr, stream))
+        return e;
     hipLaunchKernelGGL(k_b_init, dim3(B), dim3(kThreads), 0, stream, tb, b, static_cast<const double*>(q), r, p, rr,
                        bb);
     hipLaunchKernelGGL(k_b_init_state, dim3(1), dim3(64), 0, stream, st, sa, tb, static_cast<const double*>(rr),

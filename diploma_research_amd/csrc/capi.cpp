@@ -830,8 +830,7 @@ dim_status dim_csr5_spmv_transpose(const dim_csr5* A, dim_dtype dtype, const voi
         return st;
     if ((A->f.rows && !x) || (A->f.cols && !y))
         return fail(DIM_INVALID_ARGUMENT, "null vector");
-    DIM_HIP_TRY(launch_spmv_transpose(A->f, dtype == DIM_F32, x, y, static_cast<hipStream_t>(stream)));
-    return DIM_SUCCESS;
+    return launch_spmv_transpose(const_cast<dim_csr5*>(A), dtype == DIM_F32, x, y, static_cast<hipStream_t>(stream));
 }
 
 dim_status dim_csr5_sampled_outer(const dim_csr5* A, double scale, const double* u, const double* v, double* out,

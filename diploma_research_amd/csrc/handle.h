@@ -23,6 +23,17 @@ struct SystemTiles {
     uint32_t tile0, tile1;
     uint64_t nnz0, nnz;
 };
+// Where the products of y = A^T x go before they are summed (transpose.hip):
+// workgroup b (tiles [b * per, (b + 1) * per)) writes its products of columns
+// [bin << shift, (bin + 1) << shift) from place start[bin] + off[b * bins + bin] on.
+struct TransposePlan {
+    uint32_t shift = 0, bins = 0, per = 0, blocks = 0; // bins == 0: no plan
+    uint32_t* off = nullptr;
+    uint32_t* start = nullptr; // bins + 1
+    void* prod = nullptr;      // a product per element, FP64-sized
+    uint16_t* col = nullptr;   // and its column within the bin
+    bool refused = false;      // the matrix keeps the atomics
+};
 } // namespace dimgpu
 
 struct dim_csr5 {
@@ -46,6 +57,7 @@ struct dim_csr5 {
     uint64_t nnz_logical = 0; // stored elements (the format's nnz counts padding inside a batch)
     dimgpu::BoundaryInfo binfo; // host copy of the tile flags (f.binfo points here)
     dimgpu::DiaForm dia;        // stencil matrices: the values by diagonal (dia.h)
+    dimgpu::TransposePlan tplan; // made with the first transposed product
     // Column slices for plain products (capi.cpp): xs is the matrix whose
     // rows are the (column slice s, row i) pairs that hold elements, in the
     // order of s*rows + i. That stacked handle also owns the partial products
@@ -130,6 +142,10 @@ hipError_t launch_set_values(const dim_csr5* h, const double* vals_csr, hipStrea
 // out[e] = scale * u[row(e)] * v[col(e)] for every stored element e, in CSR order.
 hipError_t launch_sampled_outer(const dim_csr5* h, double scale, const double* u, const double* v, double* out,
                                 hipStream_t stream);
+
+// y = A^T x (x has rows entries, y has cols entries). done: as launch_spmv.
+dim_status launch_spmv_transpose(dim_csr5* h, bool f32, const void* x, void* y, hipStream_t stream,
+                                 const int* done = nullptr);
 
 // Writes the values of the diagonal form from the tile layout. The places
 // without an element are not written: they must hold 0.

@@ -113,10 +113,6 @@ hipError_t launch_spmv(const DevFormat& A, Scratch& S, bool f32, int k, const vo
 hipError_t launch_spmv_events(const DevFormat& A, Scratch& S, bool f32, const void* x, void* y, hipEvent_t e0,
                               hipEvent_t e1, hipEvent_t e2, hipStream_t stream, bool* fixup_launched = nullptr);
 
-// y = A^T x (x has rows entries, y has cols entries); y is zeroed first.
-hipError_t launch_spmv_transpose(const DevFormat& A, bool f32, const void* x, void* y, hipStream_t stream,
-                                 const int* done = nullptr);
-
 // y[i] = sum over the column slices s = 0..slices-1, in that order, of the
 // partial product of (s, i): the partials of the pairs whose bit s*rows + i
 // is set in `present`, stored at the rank of that bit (rank[w] = set bits

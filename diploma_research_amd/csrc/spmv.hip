@@ -28,52 +28,6 @@ namespace {
 
 using namespace detail;
 
-// ------------------------------------------------------ transpose SpMV ---
-
-template<typename V>
-__global__ void k_fill(V* y, size_t n, V value, const int* done) {
-    if (done && *done)
-        return;
-    for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        y[i] = value;
-}
-
-// y[col] += a_ij * x[row] for every element: the transposed product scatters
-// into y with hardware floating-point atomics.
-template<typename V, int SIGMA>
-__global__ __launch_bounds__(256) void k_csr5_transpose(TileParams p) {
-    if (p.done && *p.done)
-        return;
-    const int lane = threadIdx.x & 63;
-    const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= p.tile_end)
-        return;
-    using W = typename DescWord<SIGMA>::type;
-    const V* x = static_cast<const V*>(p.x);
-    V* y = static_cast<V*>(p.y);
-    const size_t base = static_cast<size_t>(t) * (64 * SIGMA);
-    const uint32_t bits = static_cast<uint32_t>(static_cast<const W*>(p.bit_flag)[static_cast<size_t>(t) * 64 + lane]) |
-                          (lane == 0 ? 1u : 0u);
-    const uint32_t tpw = p.tile_ptr[t];
-    const bool dirty = (tpw & kDirty) != 0;
-    const uint32_t row0 = tpw & ~kDirty;
-    const uint32_t* tdo = dirty ? p.tdo + p.tdo_ptr[t] : nullptr;
-    const int nb = __popc(bits);
-    const int y_off = wave_incl_scan(nb, lane) - nb;
-    const V* vals = static_cast<const V*>(p.vals);
-#pragma unroll
-    for (int r = 0; r < SIGMA; ++r) {
-        const size_t pos = base + static_cast<size_t>(r) * 64 + lane;
-        const size_t csr = base + static_cast<size_t>(lane) * SIGMA + r;
-        if (csr >= p.nnz)
-            continue;
-        const uint32_t row = element_row(bits, r, y_off, row0, dirty, tdo);
-        const V a = vals[pos];
-        unsafeAtomicAdd(y + p.col_idx[pos], a * x[row]);
-    }
-}
-
 TileParams make_tile_params(const DevFormat& A, bool f32) {
     TileParams tp{};
     tp.tile_ptr = A.tile_ptr;
@@ -427,36 +381,6 @@ hipError_t launch_slice_sum(bool f32, const void* ystack, const uint32_t* presen
     else
         hipLaunchKernelGGL((k_slice_sum<double, 8>), dim3(grid), dim3(256), 0, stream,
                            static_cast<const double*>(ystack), present, rank, rows, static_cast<double*>(y));
-    return hipGetLastError();
-}
-
-hipError_t launch_spmv_transpose(const DevFormat& A, bool f32, const void* x, void* y, hipStream_t stream,
-                                 const int* done) {
-    TileParams tp = make_tile_params(A, f32);
-    tp.x = x;
-    tp.y = y;
-    tp.done = done;
-    const uint32_t fill_grid = 1024;
-    if (f32)
-        hipLaunchKernelGGL(k_fill<float>, dim3(fill_grid), dim3(256), 0, stream, static_cast<float*>(y),
-                           static_cast<size_t>(A.cols), 0.0f, done);
-    else
-        hipLaunchKernelGGL(k_fill<double>, dim3(fill_grid), dim3(256), 0, stream, static_cast<double*>(y),
-                           static_cast<size_t>(A.cols), 0.0, done);
-    if (A.tiles) {
-        const uint32_t grid = (A.tiles + 3) / 4;
-#define DIM_T_F(S)                                                                                                    \
-    case S: hipLaunchKernelGGL((k_csr5_transpose<float, S>), dim3(grid), dim3(256), 0, stream, tp); break;
-#define DIM_T_D(S)                                                                                                    \
-    case S: hipLaunchKernelGGL((k_csr5_transpose<double, S>), dim3(grid), dim3(256), 0, stream, tp); break;
-        if (f32) {
-            switch (A.sigma) { DIM_FOR_EACH_SIGMA(DIM_T_F) default: break; }
-        } else {
-            switch (A.sigma) { DIM_FOR_EACH_SIGMA(DIM_T_D) default: break; }
-        }
-#undef DIM_T_F
-#undef DIM_T_D
-    }
     return hipGetLastError();
 }
 
