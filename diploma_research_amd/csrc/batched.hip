@@ -863,7 +863,7 @@ dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32
     // (only where the resident solver takes the batch)
     if (dia_nd && resident_batch(sys_row, f.dia_off, dia_nd).ok) {
         DiaForm D;
-        DIM_HIP_TRY(alloc_diagonals(h, dia_nd, D));
+        DIM_HIP_TRY(alloc_diagonals(h, dia_nd, 0, D));
         if (D.nd) {
             int32_t* off = nullptr;
             DIM_HIP_TRY(upload(h, off, f.dia_off));

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <random>
 #include <string>
 
@@ -31,6 +32,66 @@ dim_status hip_fail(hipError_t e, const char* what) {
     return e == hipErrorOutOfMemory ? DIM_OUT_OF_MEMORY : DIM_HIP_ERROR;
 }
 
+namespace {
+struct KeptBlock {
+    std::mutex m;
+    void* p = nullptr;
+    size_t bytes = 0;
+};
+constexpr int kMaxDevices = 64;
+KeptBlock g_kept[kMaxDevices];
+constexpr size_t kKeepMin = size_t{16} << 20, kKeepMax = size_t{256} << 20;
+
+int current_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices ? dev : -1;
+}
+} // namespace
+
+bool drop_block() {
+    const int dev = current_device();
+    if (dev < 0)
+        return false;
+    KeptBlock& k = g_kept[dev];
+    std::lock_guard<std::mutex> g(k.m);
+    if (!k.p)
+        return false;
+    (void)hipFree(k.p);
+    k.p = nullptr;
+    return true;
+}
+
+hipError_t take_block(size_t bytes, void** p, size_t* got) {
+    const int dev = current_device();
+    if (dev >= 0 && bytes >= kKeepMin) {
+        KeptBlock& k = g_kept[dev];
+        std::lock_guard<std::mutex> g(k.m);
+        if (k.p && k.bytes >= bytes && k.bytes - bytes <= bytes / 4) {
+            *p = k.p;
+            *got = k.bytes;
+            k.p = nullptr;
+            return hipSuccess;
+        }
+        if (k.p) {
+            (void)hipFree(k.p);
+            k.p = nullptr;
+        }
+    }
+    *got = bytes;
+    return malloc_or_drop(p, bytes);
+}
+
+void give_block(int device, void* p, size_t bytes) {
+    if (device >= 0 && device < kMaxDevices && bytes >= kKeepMin && bytes <= kKeepMax) {
+        KeptBlock& k = g_kept[device];
+        std::lock_guard<std::mutex> g(k.m);
+        std::swap(k.p, p);
+        k.bytes = bytes;
+    }
+    if (p)
+        (void)hipFree(p);
+}
+
 void free_handle(dim_csr5* h) {
     if (!h)
         return;
@@ -41,26 +102,29 @@ void free_handle(dim_csr5* h) {
     free_batch_cache(h->batch_cache);
     for (void* p : h->allocations)
         (void)hipFree(p);
+    if (h->block) {
+        (void)hipDeviceSynchronize(); // (as hipFree does)
+        give_block(h->device, h->block, h->block_bytes);
+    }
     (void)hipSetDevice(prev);
     free_handle(h->xs);
     delete h;
 }
 
-hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, DiaForm& D) {
+hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, size_t meta, DiaForm& D) {
     D.rows = h->f.rows;
     D.cols = h->f.cols;
     D.ld = (uint64_t{h->f.rows} + 63) / 64 * 64; // every diagonal starts on a 512-byte line
     const size_t n = size_t{nd} * D.ld;
-    const size_t kept = h->allocations.size();
-    const uint64_t kept_bytes = h->device_bytes;
-    hipError_t e = dev_alloc(h, D.v64, n);
-    if (e == hipSuccess && h->f.vals32)
-        e = dev_alloc(h, D.v32, n);
+    Arena keep;
+    keep.add(D.v64, n);
+    if (h->f.vals32)
+        keep.add(D.v32, n);
+    if (meta)
+        keep.add(D.meta, meta);
+    hipError_t e = keep.commit(h);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        for (; h->allocations.size() > kept; h->allocations.pop_back())
-            (void)hipFree(h->allocations.back());
-        h->device_bytes = kept_bytes;
         D = DiaForm{};
         return hipSuccess;
     }
@@ -76,9 +140,9 @@ hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, DiaForm& D) {
 // without: its products then run the tile kernels.
 static hipError_t upload_diagonals(const HostFormat& f, dim_csr5* h, bool products) {
     DiaForm D;
-    hipError_t e = alloc_diagonals(h, f.dia_nd, D);
+    hipError_t e = alloc_diagonals(h, f.dia_nd, f.dia_meta.size(), D);
     if (e == hipSuccess && D.nd)
-        e = upload(h, D.meta, f.dia_meta);
+        e = hipMemcpy(D.meta, f.dia_meta.data(), f.dia_meta.size() * sizeof(uint16_t), hipMemcpyHostToDevice);
     if (e != hipSuccess || !D.nd)
         return e;
     std::copy(f.dia_off.begin(), f.dia_off.end(), D.off);
@@ -100,55 +164,70 @@ dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, boo
     d.padded = f.padded;
     d.any_dirty = f.any_dirty;
     d.n_empty = static_cast<uint32_t>(f.empty_rows.size());
-    DIM_HIP_TRY(upload(h.get(), d.tile_ptr, f.tile_ptr));
-    if (f.sigma <= 16) {
-        std::vector<uint16_t> narrow(f.bit_flag.begin(), f.bit_flag.end());
-        uint16_t* p = nullptr;
-        DIM_HIP_TRY(upload(h.get(), p, narrow));
-        d.bit_flag = p;
-    } else {
-        uint32_t* p = nullptr;
-        DIM_HIP_TRY(upload(h.get(), p, f.bit_flag));
-        d.bit_flag = p;
+    // one allocation for everything, then the copies
+    const bool narrow = f.sigma <= 16;
+    const bool codes = !f.col_dict.empty() && !plain_columns;
+    std::vector<uint16_t> bits16;
+    if (narrow)
+        bits16.assign(f.bit_flag.begin(), f.bit_flag.end());
+    // flag words are read 4 bytes at a time: pad to a multiple of 4 plus 4
+    std::vector<uint8_t> flags(f.tile_flags);
+    flags.resize((flags.size() + 3) / 4 * 4 + 4, 0);
+    std::vector<float> v32;
+    if (keep_f32)
+        v32.assign(f.vals.begin(), f.vals.end());
+    std::vector<int32_t> dict(f.col_dict);
+    dict.resize(kMaxDiagonals, 0);
+    Arena keep;
+    uint16_t* d16 = nullptr;
+    uint32_t* d32 = nullptr;
+    keep.add(d.col_idx, f.col_idx.size());
+    keep.add(d.vals64, f.vals.size());
+    if (keep_f32)
+        keep.add(d.vals32, v32.size());
+    if (narrow)
+        keep.add(d16, bits16.size());
+    else
+        keep.add(d32, f.bit_flag.size());
+    keep.add(d.tile_ptr, f.tile_ptr.size());
+    keep.add(d.tile_flags, flags.size());
+    keep.add(d.tile_desc_offset_ptr, f.tile_desc_offset_ptr.size());
+    keep.add(d.tile_desc_offset, f.tile_desc_offset.size());
+    keep.add(d.empty_rows, f.empty_rows.size());
+    if (codes) {
+        keep.add(d.col_dict, dict.size());
+        keep.add(d.col_code, f.col_code.size());
     }
-    {
-        // flag words are read 4 bytes at a time: pad to a multiple of 4 plus 4
-        std::vector<uint8_t> flags(f.tile_flags);
-        flags.resize((flags.size() + 3) / 4 * 4 + 4, 0);
-        DIM_HIP_TRY(upload(h.get(), d.tile_flags, flags));
-    }
+    add_scratch(keep, h->s, f.tiles);
+    DIM_HIP_TRY(keep.commit_block(h.get()));
+    d.bit_flag = narrow ? static_cast<void*>(d16) : d32;
+    const auto copy = [](auto* to, const auto& from) {
+        return from.empty() ? hipSuccess
+                            : hipMemcpy(to, from.data(), from.size() * sizeof(from[0]), hipMemcpyHostToDevice);
+    };
+    DIM_HIP_TRY(copy(d.col_idx, f.col_idx));
+    DIM_HIP_TRY(copy(d.vals64, f.vals));
+    if (keep_f32)
+        DIM_HIP_TRY(copy(d.vals32, v32));
+    if (narrow)
+        DIM_HIP_TRY(copy(d16, bits16));
+    else
+        DIM_HIP_TRY(copy(d32, f.bit_flag));
+    DIM_HIP_TRY(copy(d.tile_ptr, f.tile_ptr));
+    DIM_HIP_TRY(copy(d.tile_flags, flags));
     h->binfo.assign(f.tile_flags);
     d.binfo = &h->binfo;
-    DIM_HIP_TRY(upload(h.get(), d.tile_desc_offset_ptr, f.tile_desc_offset_ptr));
-    DIM_HIP_TRY(upload(h.get(), d.tile_desc_offset, f.tile_desc_offset));
-    DIM_HIP_TRY(upload(h.get(), d.col_idx, f.col_idx));
-    DIM_HIP_TRY(upload(h.get(), d.vals64, f.vals));
-    if (keep_f32) {
-        std::vector<float> v32(f.vals.begin(), f.vals.end());
-        DIM_HIP_TRY(upload(h.get(), d.vals32, v32));
+    DIM_HIP_TRY(copy(d.tile_desc_offset_ptr, f.tile_desc_offset_ptr));
+    DIM_HIP_TRY(copy(d.tile_desc_offset, f.tile_desc_offset));
+    DIM_HIP_TRY(copy(d.empty_rows, f.empty_rows));
+    if (codes) {
+        DIM_HIP_TRY(copy(d.col_dict, dict));
+        DIM_HIP_TRY(copy(d.col_code, f.col_code));
     }
-    DIM_HIP_TRY(upload(h.get(), d.empty_rows, f.empty_rows));
-    if (!f.col_dict.empty() && !plain_columns) {
-        std::vector<int32_t> dict(f.col_dict);
-        dict.resize(kMaxDiagonals, 0);
-        DIM_HIP_TRY(upload(h.get(), d.col_dict, dict));
-        DIM_HIP_TRY(upload(h.get(), d.col_code, f.col_code));
-    }
+    DIM_HIP_TRY(copy(h->s.queue, std::vector<uint32_t>(kQueueWords, 0u)));
     for (uint32_t t = 0; t < f.tiles; ++t)
         h->n_dirty += (f.tile_ptr[t] & kDirty) ? 1 : 0;
 
-    Scratch& s = h->s;
-    const size_t T = std::max<size_t>(f.tiles, 1);
-    double* hp = nullptr;
-    double* tp = nullptr;
-    DIM_HIP_TRY(dev_alloc(h.get(), hp, T * kMaxK));
-    DIM_HIP_TRY(dev_alloc(h.get(), tp, T * kMaxK));
-    s.head = hp;
-    s.tail = tp;
-    DIM_HIP_TRY(dev_alloc(h.get(), s.chunk_flags, T));
-    DIM_HIP_TRY(dev_alloc(h.get(), s.dot_chunk, T * kMaxK));
-    DIM_HIP_TRY(dev_alloc(h.get(), s.dot_blk, ((T + 255) / 256) * kMaxK));
-    DIM_HIP_TRY(upload(h.get(), s.queue, std::vector<uint32_t>(kQueueWords, 0u)));
     h->sys_row = {0, f.rows};
     h->sys_tile = {0, f.tiles};
     h->sys_nnz_csr = {0, f.nnz};

@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -43,6 +45,8 @@ struct dim_csr5 {
     uint32_t n_dirty = 0;
     uint64_t device_bytes = 0;
     std::vector<void*> allocations;
+    void* block = nullptr; // the arrays of the format and the scratch (take_block)
+    size_t block_bytes = 0;
     // block-diagonal batches: system i owns rows [sys_row[i], sys_row[i+1]) and
     // tiles [sys_tile[i], sys_tile[i+1])
     uint32_t n_systems = 1;
@@ -104,19 +108,108 @@ dim_status stage_host_vectors(dim_csr5* A, char** x, char** y);
             return ::dimgpu::hip_fail(e_, #expr);                                                                  \
     } while (0)
 
+// The block of a handle's arrays. Allocating and freeing one of more than 64 MB
+// costs 0.35 ms (a program that converts matrix after matrix spends more on it
+// than on the conversion, and after a thousand of them 2 ms each), so the last
+// one freed, if it is between 16 and 256 MiB, is kept for the next conversion:
+// one block per device, freed when the next request does not fit it, when
+// another takes its place, or when an allocation of the library finds no room.
+// give_block() expects that no work on the block is in flight.
+hipError_t take_block(size_t bytes, void** p, size_t* got);
+void give_block(int device, void* p, size_t bytes);
+// Frees the current device's kept block; false if there is none.
+bool drop_block();
+
+// hipMalloc that gives up the kept block before it fails.
+inline hipError_t malloc_or_drop(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && drop_block()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 // device allocation owned by the handle
 template<typename T>
 hipError_t dev_alloc(dim_csr5* h, T*& p, size_t count) {
     p = nullptr;
     const size_t bytes = count ? count * sizeof(T) : sizeof(T);
     void* q = nullptr;
-    hipError_t e = hipMalloc(&q, bytes);
+    hipError_t e = malloc_or_drop(&q, bytes);
     if (e != hipSuccess)
         return e;
     h->allocations.push_back(q);
     h->device_bytes += bytes;
     p = static_cast<T*>(q);
     return hipSuccess;
+}
+
+// Several device arrays in one allocation, each on a 256-byte boundary: add()
+// them, then commit() once.
+class Arena {
+  public:
+    template<typename T>
+    void add(T*& p, size_t count) {
+        p = nullptr;
+        parts_.push_back({[&p](char* at) { p = reinterpret_cast<T*>(at); }, bytes_});
+        bytes_ += (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    void add_bytes(void*& p, size_t bytes) {
+        p = nullptr;
+        parts_.push_back({[&p](char* at) { p = at; }, bytes_});
+        bytes_ += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+    }
+    // the caller frees *base
+    hipError_t commit(void** base) {
+        *base = nullptr;
+        const hipError_t e = malloc_or_drop(base, std::max<size_t>(bytes_, 1));
+        if (e == hipSuccess)
+            place(*base);
+        return e;
+    }
+    // the handle frees it
+    hipError_t commit(dim_csr5* h) {
+        void* base = nullptr;
+        const hipError_t e = commit(&base);
+        if (e == hipSuccess) {
+            h->allocations.push_back(base);
+            h->device_bytes += bytes_;
+        }
+        return e;
+    }
+    // as the handle's block
+    hipError_t commit_block(dim_csr5* h) {
+        const hipError_t e = take_block(std::max<size_t>(bytes_, 1), &h->block, &h->block_bytes);
+        if (e == hipSuccess) {
+            place(h->block);
+            h->device_bytes += bytes_;
+        }
+        return e;
+    }
+
+  private:
+    void place(void* base) {
+        for (const Part& p : parts_)
+            p.set(static_cast<char*>(base) + p.at);
+    }
+    struct Part {
+        std::function<void(char*)> set;
+        size_t at;
+    };
+    std::vector<Part> parts_;
+    size_t bytes_ = 0;
+};
+
+// The products' scratch for a matrix of T tiles (the queue must be cleared).
+inline void add_scratch(Arena& a, Scratch& s, uint32_t T) {
+    const size_t n = std::max<size_t>(T, 1);
+    a.add_bytes(s.head, n * kMaxK * sizeof(double));
+    a.add_bytes(s.tail, n * kMaxK * sizeof(double));
+    a.add(s.chunk_flags, n);
+    a.add(s.dot_chunk, n * kMaxK);
+    a.add(s.dot_blk, ((n + 255) / 256) * kMaxK);
+    a.add(s.queue, kQueueWords);
 }
 
 template<typename T>
@@ -152,7 +245,8 @@ dim_status launch_spmv_transpose(dim_csr5* h, bool f32, const void* x, void* y, 
 hipError_t launch_dia_fill(const dim_csr5* h, hipStream_t stream);
 
 // Device memory of a diagonal form with nd diagonals (values zeroed, FP32 ones
-// if the handle keeps them); hipSuccess with D.nd == 0 when there is no room.
-hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, DiaForm& D);
+// if the handle keeps them) and `meta` row words; hipSuccess with D.nd == 0 when
+// there is no room.
+hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, size_t meta, DiaForm& D);
 
 } // namespace dimgpu
