@@ -336,20 +336,26 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
     // right-hand side inside the tile, after the decode.
     constexpr bool XREG = KMAX == 1;
     constexpr bool REG = XREG || SIGMA <= kSmmRegSigma;
-    // Plain single-vector products stage the row sums of a clean tile's
-    // general path in LDS (one region per wavefront of the 256-thread block)
-    // and write the tile's rows with one coalesced pass: written where they
-    // are closed, the sums of short rows reach y as scattered 8-byte stores
-    // that fill each line of y piecemeal. Measured on the MI355X, power-law
-    // product (column-sliced, 2.5 elements per stacked row): those stores
-    // took 135 of its 596 us.
-    constexpr bool STAGE = KMAX == 1 && !DOT && SIGMA <= 8;
+    // Plain single-vector products stage a tile's row sums (general path) in
+    // LDS, one region per wavefront of the 256-thread block, and write the
+    // tile's rows in one pass. Written where they are closed, the sums of
+    // short rows reach y as scattered 8-byte stores that fill each line of y
+    // piecemeal, and in a tile with empty rows every step that closes a row
+    // waits for the row's number from memory (8.2M elements, uneven rows of 12
+    // on average, 2% empty, sigma 16: 67.9 us without, 56.9 with).
+    constexpr bool STAGE = KMAX == 1 && !DOT;
     V* ystage = nullptr;
     if constexpr (STAGE) {
         __shared__ V ybuf[4][64 * SIGMA];
         ystage = ybuf[(threadIdx.x >> 6) & 3];
     }
     constexpr bool PIPE = XREG && SIGMA <= 8;
+    // Taller tiles have the next tile's column indices in flight, so that a
+    // tile's gathers start with its values' loads (the product above: 56.9 ->
+    // 54.4 us). Three wavefronts per SIMD instead of two (155 VGPRs instead of
+    // 172, the next columns always loaded): 60.5 us, the gathers then push
+    // one another's x out of L1.
+    constexpr bool COLS_AHEAD = XREG && !PIPE;
     constexpr bool CODED = CODES && REG && SIGMA <= 8;
     // The dot needs x at every row the product writes. A coded single-vector
     // product takes it from its own gathers where it can: the element on the
@@ -386,20 +392,23 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
     // they take the base from scalar registers (the readfirstlane keeps the
     // compiler from turning the bases into per-lane 64-bit pointers).
     const uint32_t ulane = static_cast<uint32_t>(lane);
-    auto fetch = [&](uint32_t t, Stage& s) {
-        const size_t tile64 = static_cast<size_t>(__builtin_amdgcn_readfirstlane(t)) * 64;
-        const size_t base = tile64 * SIGMA;
+    auto fetch_vals = [&](uint32_t t, Stage& s) {
         if constexpr (REG) {
-            const V* vt = vals_all + base;
-            const uint32_t* ct = p.col_idx + base;
+            const V* vt = vals_all + static_cast<size_t>(__builtin_amdgcn_readfirstlane(t)) * (64 * SIGMA);
 #pragma unroll
-            for (int r = 0; r < SIGMA; ++r) {
+            for (int r = 0; r < SIGMA; ++r)
                 s.v[r] = ldg_stream<NT>(vt + r * 64 + ulane);
-                if constexpr (!CODED)
-                    s.col[r] = ldg_stream<NT>(ct + r * 64 + ulane);
-            }
-            if constexpr (CODED)
-                s.code = ldg_stream<NT>(p.col_code + tile64 + ulane);
+        }
+    };
+    auto fetch_cols = [&](uint32_t t, Stage& s) {
+        const size_t tile64 = static_cast<size_t>(__builtin_amdgcn_readfirstlane(t)) * 64;
+        if constexpr (REG && CODED) {
+            s.code = ldg_stream<NT>(p.col_code + tile64 + ulane);
+        } else if constexpr (REG) {
+            const uint32_t* ct = p.col_idx + tile64 * SIGMA;
+#pragma unroll
+            for (int r = 0; r < SIGMA; ++r)
+                s.col[r] = ldg_stream<NT>(ct + r * 64 + ulane);
         }
         if constexpr (!CODED) // a code word carries its lane's flags
             s.bits = (bits_all + tile64)[ulane];
@@ -408,6 +417,10 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
         s.tdo_at = CODED ? 0u : sload(p.tdo_ptr + t); // coded matrices have no dirty tiles
         s.tf = sload_flag(p.tile_flags + t);
         s.tf_next = sload_flag(p.tile_flags + t + 1);
+    };
+    auto fetch = [&](uint32_t t, Stage& s) {
+        fetch_vals(t, s);
+        fetch_cols(t, s);
     };
     // Columns of a coded tile (the code word also carries the lane's row-start
     // flags): the element at step r of a lane belongs to row
@@ -455,6 +468,8 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
     Stage nx, nx2;
     if constexpr (PIPE)
         fetch(t0, nx);
+    else if constexpr (COLS_AHEAD)
+        fetch_cols(t0, nx);
 
     // How the chunk ends follows from two tile flags: it ends inside a row
     // (end_open) unless its last tile's last element ends a row; with
@@ -548,14 +563,18 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
                 fetch(t + AHEAD, slot);
             else if (LOOK && end_look && t + AHEAD == t1)
                 fetch_look(slot);
+        } else if constexpr (COLS_AHEAD) {
+            cu = slot;
+            fetch_vals(t, cu);
+#pragma unroll
+            for (int r = 0; r < SIGMA; ++r)
+                xg[r] = x[cu.col[r]];
+            __builtin_amdgcn_sched_barrier(0);
+            if (t + 1 < t1)
+                fetch_cols(t + 1, slot);
         } else {
             fetch(t, cu);
             decode(cu);
-            if constexpr (XREG) {
-#pragma unroll
-                for (int r = 0; r < SIGMA; ++r)
-                    xg[r] = x[cu.col[r]];
-            }
         }
 
         const uint32_t bits = static_cast<uint32_t>(cu.bits) | (lane == 0 ? 1u : 0u);
@@ -829,11 +848,11 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
                 for (int i = 0; i < GG; ++i)
                     seg0.a[i] = V(0);
                 auto emit = [&](int s, const Vec& val) {
-                    if (s == 0 && !starts_row) {
+                    if constexpr (STAGE) {
+                        ystage[s] = val.a[0];
+                    } else if (s == 0 && !starts_row) {
                         own0 = true;
                         seg0 = val;
-                    } else if constexpr (STAGE && !DIRTY) {
-                        ystage[s] = val.a[0];
                     } else {
                         write_row(row_of(s), val);
                     }
@@ -924,7 +943,16 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
                     emit(y_off - 1, tot);
                 }
 
-                if (!starts_row && nseg > 1) {
+                if constexpr (STAGE) {
+                    // The wave barriers keep the compiler from moving these
+                    // LDS accesses across the other lanes' stores and the next
+                    // tile's; a wavefront's LDS instructions run in order.
+                    __builtin_amdgcn_wave_barrier();
+                    if (!starts_row && nseg > 1 && lane == 0) {
+                        seg0.a[0] = ystage[0];
+                        close_carried(seg0);
+                    }
+                } else if (!starts_row && nseg > 1) {
                     // exactly one lane closed segment 0
                     const int o = __ffsll(static_cast<long long>(__ballot(own0))) - 1;
                     Vec s0;
@@ -974,20 +1002,17 @@ __device__ __forceinline__ double csr5_chunk(const TileParams& p, const uint32_t
                             carry[g + i] = tv.a[i];
                     }
                 }
-                if constexpr (STAGE && !DIRTY) {
+                if constexpr (STAGE) {
                     // Every segment in [s_lo, s_hi] was emitted exactly once
                     // (segment 0 of a tile that continues a row went to the
                     // carry or the head slot instead; the last segment stays
                     // open unless the tile completes it): write them in order.
-                    // The wave barriers keep the compiler from moving these
-                    // LDS accesses across the other lanes' stores and the next
-                    // tile's; a wavefront's LDS instructions run in order.
                     __builtin_amdgcn_wave_barrier();
                     const int s_lo = starts_row ? 0 : 1;
                     const int s_hi = complete ? nseg - 1 : nseg - 2;
                     V* yrow = y + static_cast<size_t>(row0 - p.row_base);
                     for (int i = s_lo + lane; i <= s_hi; i += 64)
-                        yrow[i] = ystage[i];
+                        yrow[DIRTY ? tdo[i] : static_cast<uint32_t>(i)] = ystage[i];
                     __builtin_amdgcn_wave_barrier();
                 }
             }
