@@ -377,6 +377,25 @@ dim_status build_slices(const StackedCsr& sc, uint32_t cols, uint32_t sigma, boo
     return DIM_SUCCESS;
 }
 
+bool windowed(const dim_csr5* h, bool f32) {
+    return (f32 ? h->win.f32 : h->win.f64).blocks != 0;
+}
+
+// The windows of a matrix built on the host. (Column codes need no column
+// indices from memory, which weighs more than the windows; matrices told to
+// keep plain columns keep the tile kernel.)
+dim_status plan_windows(dim_csr5* h, const std::vector<uint8_t>& tile_flags) {
+    const DevFormat& A = h->f;
+    if (A.col_code || h->dia.products || A.tiles < kWindowMinTiles || A.sigma > kWindowMaxSigma)
+        return DIM_SUCCESS;
+    std::vector<uint32_t> span(2 * ((A.tiles + kWindowGroup - 1) / kWindowGroup));
+    DIM_HIP_TRY(dev_alloc(h, h->win.span, span.size()));
+    DIM_HIP_TRY(launch_spans(A, h->win.span, nullptr));
+    DIM_HIP_TRY(hipMemcpy(span.data(), h->win.span, span.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    shape_windows(h, span, tile_flags);
+    return DIM_SUCCESS;
+}
+
 // The whole-matrix single-vector product, through the column slices when the
 // matrix has them.
 hipError_t plain_product(dim_csr5* h, bool f32, const void* x, void* y, hipStream_t st) {
@@ -390,6 +409,8 @@ hipError_t plain_product(dim_csr5* h, bool f32, const void* x, void* y, hipStrea
     }
     if (h->dia.products)
         return launch_dia_spmv(h->dia, f32, x, y, st);
+    if (windowed(h, f32))
+        return launch_window_spmv(h->f, h->win, f32, x, y, st);
     return launch_spmv(h->f, h->s, f32, 1, x, y, 0, h->f.tiles, 0, 0, h->f.n_empty, false, nullptr, st);
 }
 
@@ -606,6 +627,11 @@ dim_status dim_csr5_from_csr(uint32_t rows, uint32_t cols, uint64_t nnz, const u
             return st;
         }
         h->xs_slices = kXcdSlices;
+    } else if (!plain_columns) {
+        if (dim_status st = plan_windows(h, f.tile_flags)) {
+            free_handle(h);
+            return st;
+        }
     }
     *out = h;
     return DIM_SUCCESS;
@@ -746,12 +772,12 @@ dim_status dim_csr5_spmv_timed(const dim_csr5* A, dim_dtype dtype, const void* x
         if (e == hipSuccess)
             e = hipEventRecord(ev[2], st);
         fixup = true;
-    } else if (self->dia.products) {
+    } else if (self->dia.products || windowed(self, dtype == DIM_F32)) {
         // one kernel
         const auto st = static_cast<hipStream_t>(stream);
         e = hipEventRecord(ev[0], st);
         if (e == hipSuccess)
-            e = launch_dia_spmv(self->dia, dtype == DIM_F32, x, y, st);
+            e = plain_product(self, dtype == DIM_F32, x, y, st);
         if (e == hipSuccess)
             e = hipEventRecord(ev[1], st);
         if (e == hipSuccess)

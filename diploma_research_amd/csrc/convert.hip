@@ -7,7 +7,8 @@
 //   1. the CSR arrays are checked and the empty rows counted;
 //   2. a tile's first row by a 64-way search in row_ptr, then its row starts by
 //      a walk over row_ptr, 64 rows at a time: bit flags, tile flags, dirty mark;
-//   3. the per-tile transpose of values and column indices, through LDS;
+//   3. the per-tile transpose of values and column indices, through LDS, and
+//      the column spans of every 16 tiles;
 //   4. only if there are empty rows: the segment -> row maps of dirty tiles (a
 //      scan of their segment counts, then the walk again) and the list of
 //      empty rows.
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(kT) void k_check(uint32_t rows, uint32_t cols, uint
 // segment offsets too.
 __global__ __launch_bounds__(kT) void k_ends(uint32_t T, uint32_t rows, uint32_t flag_bytes, bool clean,
                                              uint32_t* tile_ptr, uint8_t* tile_flags, uint32_t* tdo_ptr, uint32_t* tdo,
-                                             uint32_t* queue) {
+                                             uint32_t* queue, uint32_t* span) {
     const uint32_t tid = blockIdx.x * kT + threadIdx.x, stride = gridDim.x * kT;
     if (tid == 0) {
         tile_ptr[T] = rows;
@@ -89,6 +90,9 @@ __global__ __launch_bounds__(kT) void k_ends(uint32_t T, uint32_t rows, uint32_t
     if (clean)
         for (uint32_t i = tid; i <= T; i += stride)
             tdo_ptr[i] = 0;
+    if (span) // (the lowest and the highest column of no tiles)
+        for (uint32_t i = tid; i < 2 * ((T + kWindowGroup - 1) / kWindowGroup); i += stride)
+            span[i] = i & 1u ? 0u : 0xffffffffu;
 }
 
 // The last row r with rp[r] <= b (b < rp[rows]), found by the whole wavefront.
@@ -263,7 +267,8 @@ __global__ __launch_bounds__(64) void k_list_empty(uint32_t rows, const uint32_t
 template<int SIGMA>
 __global__ __launch_bounds__(kT) void k_transpose(uint32_t T, uint64_t nnz, const uint32_t* __restrict__ ci,
                                                   const double* __restrict__ v, uint32_t* __restrict__ ci_out,
-                                                  double* __restrict__ v_out, float* __restrict__ v32_out) {
+                                                  double* __restrict__ v_out, float* __restrict__ v32_out,
+                                                  uint32_t* span) {
     __shared__ double stage[kT / 64][64 * (SIGMA | 1)];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t t = blockIdx.x * (kT / 64) + (threadIdx.x >> 6);
@@ -280,6 +285,23 @@ __global__ __launch_bounds__(kT) void k_transpose(uint32_t T, uint64_t nnz, cons
         const uint32_t e = r * 64 + lane;
         a[r] = e < left ? v[base + e] : 0.0;
         c[r] = e < left ? ci[base + e] : 0u;
+    }
+    if (span) {
+        uint32_t l = 0xffffffffu, h = 0;
+#pragma unroll
+        for (int r = 0; r < SIGMA; ++r) {
+            l = min(l, r * 64 + lane < left ? c[r] : 0xffffffffu);
+            h = max(h, c[r]);
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            l = min(l, static_cast<uint32_t>(__shfl_xor(static_cast<int>(l), d, 64)));
+            h = max(h, static_cast<uint32_t>(__shfl_xor(static_cast<int>(h), d, 64)));
+        }
+        if (lane == 0) {
+            atomicMin(span + 2 * (t / kWindowGroup), l);
+            atomicMax(span + 2 * (t / kWindowGroup) + 1, h);
+        }
     }
 #pragma unroll
     for (int r = 0; r < SIGMA; ++r) {
@@ -367,20 +389,25 @@ dim_status convert(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t* r
     // (a dirty tile has a segment for each of its non-empty rows, and one)
     keep.add(d.tile_desc_offset, n_empty ? size_t{rows} - n_empty + T : 1);
     keep.add(d.empty_rows, n_empty);
+    const bool spans = T >= kWindowMinTiles && sigma <= kWindowMaxSigma;
+    const size_t groups = (size_t{T} + kWindowGroup - 1) / kWindowGroup;
+    if (spans)
+        keep.add(h->win.span, 2 * groups);
     add_scratch(keep, h->s, T);
     DIM_HIP_TRY(keep.commit_block(h.get()));
     d.bit_flag = bits;
 
     const dim3 tile_grid((T + kT / 64 - 1) / (kT / 64)), block(kT);
     hipLaunchKernelGGL(k_ends, dim3(n_empty ? 1 : 32), block, 0, s, T, rows, static_cast<uint32_t>(flag_bytes),
-                       n_empty == 0, d.tile_ptr, d.tile_flags, d.tile_desc_offset_ptr, d.tile_desc_offset, h->s.queue);
+                       n_empty == 0, d.tile_ptr, d.tile_flags, d.tile_desc_offset_ptr, d.tile_desc_offset, h->s.queue, h->win.span);
     if (T) {
         hipLaunchKernelGGL((k_tiles<W>), tile_grid, block, 0, s, T, rows, n32, sigma, rp, d.tile_ptr, bits,
                            d.tile_flags, nseg_dirty, counts);
         switch (sigma) {
 #define DIM_TRANSPOSE(S)                                                                                              \
     case S:                                                                                                           \
-        hipLaunchKernelGGL((k_transpose<S>), tile_grid, block, 0, s, T, nnz, ci, v, d.col_idx, d.vals64, d.vals32);   \
+        hipLaunchKernelGGL((k_transpose<S>), tile_grid, block, 0, s, T, nnz, ci, v, d.col_idx, d.vals64, d.vals32,    \
+                           h->win.span);                                                                              \
         break;
             DIM_FOR_EACH_SIGMA(DIM_TRANSPOSE)
 #undef DIM_TRANSPOSE
@@ -404,8 +431,13 @@ dim_status convert(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t* r
     DIM_HIP_TRY(hipGetLastError());
     // host copy of the tile flags for the launch planner
     std::vector<uint8_t> hflags(size_t{T} + 1);
+    std::vector<uint32_t> hspan(spans ? 2 * groups : 0);
     DIM_HIP_TRY(hipMemcpyAsync(hflags.data(), d.tile_flags, size_t{T} + 1, hipMemcpyDeviceToHost, s));
+    if (spans)
+        DIM_HIP_TRY(hipMemcpyAsync(hspan.data(), h->win.span, hspan.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     DIM_HIP_TRY(hipStreamSynchronize(s));
+    if (spans)
+        shape_windows(h.get(), hspan, hflags);
     h->binfo.assign(std::move(hflags));
     d.binfo = &h->binfo;
     d.any_dirty = got.ntdo != 0;

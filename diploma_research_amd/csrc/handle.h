@@ -5,6 +5,7 @@
 #include "dia.h"
 #include "dim_internal.h"
 #include "kernels.h"
+#include "window.h"
 #include "../../include/dim_gpu.h"
 
 #include <hip/hip_runtime.h>
@@ -35,6 +36,7 @@ struct TransposePlan {
     void* prod = nullptr;      // a product per element, FP64-sized
     uint16_t* col = nullptr;   // and its column within the bin
     bool refused = false;      // the matrix keeps the atomics
+    bool band = false;         // by windows (window.h) instead: prod holds their sums
 };
 } // namespace dimgpu
 
@@ -61,6 +63,7 @@ struct dim_csr5 {
     uint64_t nnz_logical = 0; // stored elements (the format's nnz counts padding inside a batch)
     dimgpu::BoundaryInfo binfo; // host copy of the tile flags (f.binfo points here)
     dimgpu::DiaForm dia;        // stencil matrices: the values by diagonal (dia.h)
+    dimgpu::WindowPlan win;     // matrices within a band (window.h)
     dimgpu::TransposePlan tplan; // made with the first transposed product
     // Column slices for plain products (capi.cpp): xs is the matrix whose
     // rows are the (column slice s, row i) pairs that hold elements, in the
@@ -227,6 +230,14 @@ hipError_t upload(dim_csr5* h, T*& p, const std::vector<T>& v) {
 dim_status upload_format(const HostFormat& f, bool keep_f32, dim_csr5** out, bool plain_columns = false);
 
 void free_handle(dim_csr5* h);
+
+// The windows of a matrix on the device, from its spans on the host (window.h).
+inline void shape_windows(dim_csr5* h, const std::vector<uint32_t>& span, const std::vector<uint8_t>& tile_flags) {
+    h->win.f64 = window_shape(h->f.tiles, h->f.sigma, span, tile_flags, sizeof(double));
+    h->win.sums = window_sums_shape(h->f.tiles, h->f.sigma, span);
+    if (h->f.vals32)
+        h->win.f32 = window_shape(h->f.tiles, h->f.sigma, span, tile_flags, sizeof(float));
+}
 
 // New values (CSR order) into the tile layout, FP64 and, if kept, FP32, and into
 // the diagonal form.

@@ -1,0 +1,62 @@
+// Products of matrices whose elements lie within a band (window.hip).
+#pragma once
+
+#include "dim_internal.h"
+#include "kernels.h"
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <vector>
+
+namespace dimgpu {
+
+constexpr uint32_t kWindowGroup = 16; // tiles whose column span is kept; wavefronts of a workgroup
+constexpr uint32_t kWindowMaxPer = 4;
+constexpr uint32_t kWindowMaxSigma = 16;
+constexpr uint32_t kWindowMinTiles = 1024; // 64 workgroups
+
+// How a product is cut: workgroups of 16 wavefronts with `per` tiles each, and
+// the largest window, in entries of x; blocks == 0: the tile kernel's.
+struct WindowShape {
+    uint32_t per = 0, blocks = 0, width = 0;
+};
+
+struct WindowPlan {
+    uint32_t* span = nullptr; // lowest and highest column of every 16 tiles
+    WindowShape f64, f32;
+    WindowShape sums; // of the transposed product (transpose.hip)
+};
+
+// The shape for values of vb bytes, from the spans and the tile flags (tiles + 1
+// entries).
+WindowShape window_shape(uint32_t tiles, uint32_t sigma, const std::vector<uint32_t>& span,
+                         const std::vector<uint8_t>& tile_flags, size_t vb);
+
+WindowShape window_sums_shape(uint32_t tiles, uint32_t sigma, const std::vector<uint32_t>& span);
+
+namespace detail {
+
+// The columns [lo, lo + w) of workgroup b's tiles.
+__device__ __forceinline__ void window_of(const uint32_t* span, uint32_t tiles, const WindowShape& S, uint32_t b,
+                                          uint32_t* lo, uint32_t* w) {
+    const uint32_t groups = (tiles + kWindowGroup - 1) / kWindowGroup;
+    const uint32_t g0 = b * S.per, g1 = min(g0 + S.per, groups);
+    uint32_t l = 0xffffffffu, h = 0;
+    for (uint32_t g = g0; g < g1; ++g) {
+        l = min(l, span[2 * g]);
+        h = max(h, span[2 * g + 1]);
+    }
+    *lo = l;
+    *w = min(h - l + 1u, S.width);
+}
+
+} // namespace detail
+
+hipError_t launch_spans(const DevFormat& A, uint32_t* span, hipStream_t stream);
+
+// y = A x.
+hipError_t launch_window_spmv(const DevFormat& A, const WindowPlan& P, bool f32, const void* x, void* y,
+                              hipStream_t stream);
+
+} // namespace dimgpu
