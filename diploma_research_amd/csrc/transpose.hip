@@ -7,6 +7,11 @@
 // column's bin, and the second sums each bin in LDS and writes its part of y
 // once. Where a workgroup's products of a bin go follows from the pattern
 // alone; it is counted with a matrix's first product (3 small kernels) and kept.
+//
+// Where the elements lie within a band, a workgroup's columns fit LDS and
+// nothing is sorted: it adds its products up there, writes the sums of its
+// window, and a second kernel adds the windows up (4.1M elements within a band
+// of 18000 columns, FP64: 27.6 us against 68.5 sorted).
 #include "handle.h"
 #include "spmv_impl.h"
 
@@ -18,6 +23,7 @@ namespace {
 
 using detail::DescWord;
 using detail::element_row;
+using detail::sload;
 using detail::wave_incl_scan;
 using detail::xcd_remap;
 
@@ -227,27 +233,179 @@ __global__ __launch_bounds__(kSortThreads) void k_sum_bins(TransposePlan T, uint
     }
 }
 
+// ---- matrices within a band ------------------------------------------------
+
+constexpr int kBandThreads = 64 * static_cast<int>(kWindowGroup);
+static_assert(kBandThreads == 1024, "one workgroup per CU: its window may take all of the LDS");
+
+// Workgroup b's sums of its window, to sums[b * width]. One workgroup of 16
+// wavefronts per CU; the products of one column meet in LDS in no fixed order
+// (FP64 sums, for FP32 products too).
+template<typename V, int SIGMA>
+__global__ __launch_bounds__(kBandThreads) void k_band_products(DevFormat A, const uint32_t* __restrict__ span,
+                                                                WindowShape S, const V* __restrict__ vals,
+                                                                const V* __restrict__ x, double* __restrict__ sums,
+                                                                const int* done) {
+    if (done && *done)
+        return;
+    extern __shared__ double sum[];
+    const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+    uint32_t lo, w;
+    detail::window_of(span, A.tiles, S, b, &lo, &w);
+    for (uint32_t i = threadIdx.x; i < w; i += kBandThreads)
+        sum[i] = 0.0;
+    __syncthreads();
+    const uint32_t tb = b * kWindowGroup * S.per, te = min(tb + kWindowGroup * S.per, A.tiles);
+    const int lane = threadIdx.x & 63;
+    const uint32_t ulane = static_cast<uint32_t>(lane);
+    for (uint32_t t = tb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < te; t += kWindowGroup) {
+        // (all of a tile's loads in flight together)
+        using W = typename DescWord<SIGMA>::type;
+        const size_t base = static_cast<size_t>(t) * (64 * SIGMA);
+        const uint32_t bits =
+          static_cast<uint32_t>(static_cast<const W*>(A.bit_flag)[static_cast<size_t>(t) * 64 + ulane]) |
+          (lane == 0 ? 1u : 0u);
+        uint32_t col[SIGMA], row[SIGMA];
+        V v[SIGMA], xv[SIGMA];
+#pragma unroll
+        for (int r = 0; r < SIGMA; ++r) {
+            v[r] = __builtin_nontemporal_load(vals + base + r * 64 + ulane);
+            col[r] = __builtin_nontemporal_load(A.col_idx + base + r * 64 + ulane);
+        }
+        const uint32_t tpw = sload(A.tile_ptr + t), row0 = tpw & ~kDirty;
+        const int nb = __popc(bits);
+        const uint32_t y_off = static_cast<uint32_t>(wave_incl_scan(nb, lane) - nb);
+#pragma unroll
+        for (int r = 0; r < SIGMA; ++r)
+            row[r] = y_off - 1u + static_cast<uint32_t>(__popc(bits & ((2u << r) - 1u)));
+        if (tpw & kDirty) {
+            const uint32_t* tdo = A.tile_desc_offset + sload(A.tile_desc_offset_ptr + t);
+#pragma unroll
+            for (int r = 0; r < SIGMA; ++r)
+                row[r] = tdo[row[r]];
+        }
+#pragma unroll
+        for (int r = 0; r < SIGMA; ++r)
+            xv[r] = x[row0 + row[r]];
+        const uint64_t left = A.nnz - base; // (the last tile has padding)
+#pragma unroll
+        for (int r = 0; r < SIGMA; ++r)
+            if (ulane * SIGMA + r < left)
+                unsafeAtomicAdd(sum + (col[r] - lo), static_cast<double>(v[r] * xv[r]));
+    }
+    __syncthreads();
+    double* out = sums + static_cast<size_t>(b) * S.width;
+    for (uint32_t i = threadIdx.x; i < w; i += kBandThreads)
+        out[i] = sum[i];
+}
+
+// y: every column's sums over the windows that hold it, in the workgroups'
+// order. The windows are looked through 256 at a time; those that meet the
+// workgroup's 256 columns are listed in LDS.
+template<typename V>
+__global__ __launch_bounds__(256) void k_band_sum(const uint32_t* __restrict__ span, uint32_t tiles, WindowShape S,
+                                                  uint32_t cols, const double* __restrict__ sums, V* __restrict__ y,
+                                                  const int* done) {
+    if (done && *done)
+        return;
+    __shared__ uint32_t at_s[256], lo_s[256], w_s[256], n_s[4];
+    const uint32_t c0 = blockIdx.x * 256, c = c0 + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double s = 0.0;
+    for (uint32_t b0 = 0; b0 < S.blocks; b0 += 256) {
+        const uint32_t b = b0 + threadIdx.x;
+        uint32_t lo = 0, w = 0;
+        if (b < S.blocks)
+            detail::window_of(span, tiles, S, b, &lo, &w);
+        const bool meets = lo < c0 + 256 && c0 < lo + w;
+        const uint64_t m = __ballot(meets);
+        if (lane == 0)
+            n_s[wave] = __popcll(m);
+        __syncthreads();
+        uint32_t k = __popcll(m & ((1ull << lane) - 1ull)), n = 0;
+        for (uint32_t q = 0; q < 4; ++q) {
+            k += q < wave ? n_s[q] : 0u;
+            n += n_s[q];
+        }
+        if (meets) {
+            at_s[k] = b;
+            lo_s[k] = lo;
+            w_s[k] = w;
+        }
+        __syncthreads();
+        constexpr uint32_t U = 8;
+        for (uint32_t i = 0; i < n; i += U) {
+            double v[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const uint32_t q = min(i + u, n - 1u);
+                const uint32_t o = c - lo_s[q];
+                v[u] = i + u < n && o < w_s[q] ? sums[static_cast<size_t>(at_s[q]) * S.width + o] : 0.0;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u)
+                s += v[u];
+        }
+        __syncthreads();
+    }
+    if (c < cols)
+        y[c] = static_cast<V>(s);
+}
+
+template<typename V, int SIGMA>
+hipError_t launch_band(const dim_csr5* h, const V* vals, const V* x, V* y, hipStream_t stream, const int* done) {
+    const WindowShape& S = h->win.sums;
+    const uint32_t bytes = S.width * static_cast<uint32_t>(sizeof(double));
+    const void* f = reinterpret_cast<const void*>(&k_band_products<V, SIGMA>);
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    if (e != hipSuccess)
+        return e;
+    double* sums = static_cast<double*>(h->tplan.prod);
+    hipLaunchKernelGGL((k_band_products<V, SIGMA>), dim3(S.blocks), dim3(kBandThreads), bytes, stream, h->f,
+                       static_cast<const uint32_t*>(h->win.span), S, vals, x, sums, done);
+    hipLaunchKernelGGL(k_band_sum<V>, dim3((h->f.cols + 255) / 256), dim3(256), 0, stream,
+                       static_cast<const uint32_t*>(h->win.span), h->f.tiles, S, h->f.cols,
+                       static_cast<const double*>(sums), y, done);
+    return hipGetLastError();
+}
+
+// ---- which of them ---------------------------------------------------------
+
 // The matrix's plan, made with its first product; sorted == false when it
 // keeps the atomics (few elements, very many columns, no room, or a stream
 // that is being captured before the plan exists).
 dim_status transpose_plan(dim_csr5* h, hipStream_t stream, bool* sorted) {
     const DevFormat& A = h->f;
     TransposePlan& T = h->tplan;
-    *sorted = T.bins != 0;
+    *sorted = T.bins != 0 || T.band;
     if (*sorted || T.refused || A.nnz < kSortElements)
         return DIM_SUCCESS;
+    const bool band = h->win.sums.blocks != 0;
     // about 512 bins, of 64 to 8192 columns
     uint32_t shift = 6;
     while (shift < kMaxShift && (A.cols >> shift) >= 512)
         ++shift;
     const uint32_t bins = (A.cols + (1u << shift) - 1) >> shift;
-    if (bins > kMaxBins) {
+    if (bins > kMaxBins && !band) {
         T.refused = true;
         return DIM_SUCCESS;
     }
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
+        return DIM_SUCCESS;
+    }
+    if (band) {
+        double* sums = nullptr;
+        const hipError_t e = dev_alloc(h, sums, size_t{h->win.sums.blocks} * h->win.sums.width);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            T.refused = true;
+            return DIM_SUCCESS;
+        }
+        DIM_HIP_TRY(e);
+        T.prod = sums;
+        T.band = *sorted = true;
         return DIM_SUCCESS;
     }
     TransposePlan p;
@@ -295,6 +453,16 @@ hipError_t product(const dim_csr5* h, bool sorted, const V* vals, const V* x, V*
     const DevFormat& A = h->f;
     const TransposePlan& T = h->tplan;
     // enough workgroups for the chip where the bins are few
+    if (T.band) {
+        switch (A.sigma) {
+#define DIM_B(S)                                                                                                      \
+    case S:                                                                                                           \
+        return launch_band<V, S>(h, vals, x, y, stream, done);
+            DIM_B(4) DIM_B(5) DIM_B(6) DIM_B(7) DIM_B(8) DIM_B(10) DIM_B(12) DIM_B(14) DIM_B(16)
+#undef DIM_B
+            default: return hipErrorInvalidValue;
+        }
+    }
     const uint32_t shares = sorted ? std::max(1u, 256u / T.bins) : 0u;
     if (shares != 1)
         hipLaunchKernelGGL(k_fill<V>, dim3(1024), dim3(256), 0, stream, y, static_cast<size_t>(A.cols), V(0), done);
