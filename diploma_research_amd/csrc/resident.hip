@@ -14,14 +14,18 @@
 //
 // One iteration, with two meetings of the team (reference: textbook CG,
 // thesis.tex:2133-2160):
-//   1. p = r + beta p for the own rows and for the halo (r and p of the
-//      neighbours, published in step 3); q = A p; p.q
+//   1. p = r + beta p for the own rows and for the halo (r of the neighbours,
+//      published in step 3, and the halo's p of the iteration before); q = A p;
+//      p.q
 //   -- meeting: the sum of p.q, alpha
 //   2. x += alpha p, r -= alpha q, r.r
-//   3. r and p of the rows that others read go to memory
+//   3. r of the rows that others read goes to memory
 //   -- meeting: the sum of r.r, stop test, beta
 // Every workgroup computes the halo's p itself, from the same numbers in the
-// same way as its owner, so p needs no meeting of its own.
+// same way as its owner, and keeps it, so p needs no meeting of its own and does
+// not go through memory (with p published beside r: 128^3 cells to 1e-12 16.7
+// ms, now 13.9; 256^2 cells 3.30 and 2.94 ms). Only where the registers are full
+// (far_in_registers()) a far diagonal's p comes from its owner.
 //
 // The launch is an ordinary one: a cooperative launch takes a resource that
 // only one process on the GPU can hold. Its workgroups first wait until all of
@@ -66,6 +70,13 @@ constexpr bool values_resident(uint32_t nd, uint32_t rpt, size_t vb) {
 // the loads in flight would crowd the registers.
 constexpr bool x_in_lds(uint32_t nd, uint32_t rpt, size_t vb) {
     return ((values_resident(nd, rpt, vb) ? rpt : chunk_rows(rpt)) * nd + chunk_rows(rpt) * 4 + 3 * rpt) * vb / 4 > 150;
+}
+// The direction where far diagonals reach stays in registers if there is room
+// beside r, A p, x and the values (spills set in above about these counts);
+// otherwise it is read from its owners' memory in every iteration.
+constexpr bool far_in_registers(uint32_t nd, uint32_t rpt, size_t vb) {
+    const bool res = values_resident(nd, rpt, vb);
+    return ((res ? rpt : chunk_rows(rpt)) * nd + (x_in_lds(nd, rpt, vb) ? 4 : 5) * rpt) * vb / 4 <= (res ? 165 : 190);
 }
 constexpr unsigned kCalledOff = 0x10000; // added to the seat count
 constexpr long long kEmpty = -1; // a slot nobody has written: no sum has these bits
@@ -235,8 +246,11 @@ template<typename V, int ND, int RPT, bool WIDE, bool FAR>
 __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
     constexpr bool RES = values_resident(ND, RPT, sizeof(V));
     constexpr bool XLDS = x_in_lds(ND, RPT, sizeof(V));
+    constexpr bool KEEP = FAR && far_in_registers(ND, RPT, sizeof(V));
     constexpr int CH = chunk_rows(RPT);
-    constexpr int U = 8; // halo entries per thread in flight together
+    // halo entries per thread in flight together (8 would spill beside the most
+    // resident values: 8 FP32-refined columns of 64^3 cells 12.8 ms)
+    constexpr int U = RES && RPT == 16 ? 4 : 8;
     const ResidentJob& J = a.jobs[job];
     const uint32_t n = J.rows, H = J.halo;
     const uint32_t first_row = team.tb * J.rb < n ? team.tb * J.rb : 0u;
@@ -266,6 +280,7 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
 
     V* xs = win + (RPT * kThreads + 2 * H); // x, where it lives in LDS
     V x[XLDS ? 1 : RPT], r[RPT], v[RES ? RPT : 1][ND];
+    V flo[KEEP ? RPT : 1], fhi[KEEP ? RPT : 1]; // p where the far diagonals reach
     for (uint32_t h = threadIdx.x; h < RPT * kThreads + 2 * H; h += kThreads)
         win[h] = V(0);
     __syncthreads();
@@ -310,7 +325,7 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
         }
         if (team.tn > 1 && H) {
             for (uint32_t u0 = 0; u0 < 2 * H; u0 += U * kThreads) {
-                V hr[U], hp[U];
+                V hr[U];
                 // entry h of the halo is row first_row - H + h, past the own
                 // rows from h = H on
 #pragma unroll
@@ -318,17 +333,17 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
                     const int h = static_cast<int>(u0 + u * kThreads + tid);
                     const int row = static_cast<int>(first_row) + h + (h < static_cast<int>(H) ? -static_cast<int>(H) : static_cast<int>(rows) - static_cast<int>(H));
                     const uint32_t at = static_cast<uint32_t>(max(0, min(row, static_cast<int>(n) - 1)));
-                    hr[u] = load_shared(R + at);
-                    hp[u] = load_shared(P + at);
+                    hr[u] = load_shared((fresh ? P : R) + at);
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const uint32_t h = u0 + u * kThreads + tid;
                     const int row = static_cast<int>(first_row + h) + (h < H ? -static_cast<int>(H) : static_cast<int>(rows) - static_cast<int>(H));
-                    V pv = (fresh ? V(0) : hr[u]) + beta * hp[u];
-                    pv = row >= 0 && row < static_cast<int>(n) ? pv : V(0);
-                    if (h < 2 * H)
-                        win[h < H ? h : rows + h] = pv;
+                    if (h < 2 * H) {
+                        V* w = win + (h < H ? h : rows + h);
+                        const V pv = fresh ? hr[u] : hr[u] + beta * *w;
+                        *w = row >= 0 && row < static_cast<int>(n) ? pv : V(0);
+                    }
                 }
             }
         }
@@ -343,21 +358,31 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
             if (c < nj) {
                 V plo[CH], phi[CH];
                 if constexpr (FAR) {
-                    V rlo[CH], rhi[CH];
+                    const V* from = fresh ? P : R;
+                    V qlo[KEEP ? 1 : CH], qhi[KEEP ? 1 : CH];
 #pragma unroll
                     for (int j = 0; j < CH; ++j) {
                         const int row = static_cast<int>(first_row + (c + j) * kThreads + tid);
                         const int lo = max(0, min(row + off[0], static_cast<int>(n) - 1));
                         const int hi = max(0, min(row + o_hi, static_cast<int>(n) - 1));
-                        rlo[j] = load_shared(R + lo);
-                        plo[j] = load_shared(P + lo);
-                        rhi[j] = load_shared(R + hi);
-                        phi[j] = load_shared(P + hi);
+                        plo[j] = load_shared(from + lo);
+                        phi[j] = load_shared(from + hi);
+                        if constexpr (!KEEP) {
+                            qlo[j] = load_shared(P + lo);
+                            qhi[j] = load_shared(P + hi);
+                        }
                     }
 #pragma unroll
                     for (int j = 0; j < CH; ++j) {
-                        plo[j] = (fresh ? V(0) : rlo[j]) + beta * plo[j];
-                        phi[j] = (fresh ? V(0) : rhi[j]) + beta * phi[j];
+                        if constexpr (KEEP) {
+                            plo[j] = fresh ? plo[j] : plo[j] + beta * flo[c + j];
+                            phi[j] = fresh ? phi[j] : phi[j] + beta * fhi[c + j];
+                            flo[c + j] = plo[j];
+                            fhi[c + j] = phi[j];
+                        } else {
+                            plo[j] = fresh ? plo[j] : plo[j] + beta * qlo[j];
+                            phi[j] = fresh ? phi[j] : phi[j] + beta * qhi[j];
+                        }
                     }
                 }
                 V vc[CH][ND];
@@ -419,12 +444,15 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
                 r[j] = rj;
                 acc += static_cast<double>(rj) * static_cast<double>(rj);
                 if (team.tn > 1 && l < rows && (FAR || l < H || l + H >= rows)) {
-                    if constexpr (WIDE) {
+                    if constexpr (WIDE)
                         store_chip(R + first_row + l, rj);
-                        store_chip(P + first_row + l, pj);
-                    } else {
+                    else
                         store_xcd(R + first_row + l, rj);
-                        store_xcd(P + first_row + l, pj);
+                    if constexpr (FAR && !KEEP) {
+                        if constexpr (WIDE)
+                            store_chip(P + first_row + l, pj);
+                        else
+                            store_xcd(P + first_row + l, pj);
                     }
                 }
             }
