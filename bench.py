@@ -112,6 +112,12 @@ def stream_read_ceiling(gib=4, reps=5):
     return round(best, 1)
 
 
+def by_diagonals(sigma, codes):
+    """Whether products of the 7-point operator take the diagonal form's kernel
+    (no row of 7 spans three lanes of a tile)."""
+    return codes and sigma >= 6
+
+
 def traffic_for(sigma, codes):
     """HBM bytes per launch of the headline kernel at `sigma` from the
     committed rocprofv3 FETCH_SIZE / WRITE_SIZE runs (profiles/)."""
@@ -120,7 +126,7 @@ def traffic_for(sigma, codes):
         return None
     with open(tfile) as f:
         t = json.load(f)
-    key = f"{sigma}{'c' if codes else ''}"
+    key = "dia" if by_diagonals(sigma, codes) else f"{sigma}{'c' if codes else ''}"
     entry = t.get("by_kernel", {}).get(key) or t.get("by_sigma", {}).get(str(sigma))
     return entry.get("hbm_bytes_per_launch") if entry else None
 
@@ -736,7 +742,8 @@ def main():
                    "parity_rel_err_vs_cpu_baseline": parity},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": f"k_csr5_tiles<double,{sigma},1,false,{'true' if codes else 'false'}>",
+                     "kernel": "k_dia_spmv<double,7,true>" if by_diagonals(sigma, codes) else
+                     f"k_csr5_tiles<double,{sigma},1,false,{'true' if codes else 'false'}>",
                      "kernel_ms": round(kernel_ms, 5),
                      "kernels_per_step": 1 if single_kernel else 2,
                      "kernel_ms_source": "HIP events over the timed region, one launch per step" if single_kernel
