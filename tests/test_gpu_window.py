@@ -113,3 +113,29 @@ def test_transposed_window_products(cuda, name, band, f32):
     np.testing.assert_array_equal(y.cpu().numpy().astype(np.float64), ref)
     y2 = A.spmv_transpose(to_dev(-x, torch.float32 if f32 else None), torch.full_like(y, float("nan")))
     np.testing.assert_array_equal(y2.cpu().numpy().astype(np.float64), -ref)
+
+
+def test_captured_window_products(cuda):
+    """Both products recorded and replayed with other inputs."""
+    import torch
+
+    rng = np.random.default_rng(7)
+    rp, ci, v = _matrix(_lens("uneven, some empty", 512, rng), 30000, 3000, rng)
+    rows, v = len(rp) - 1, np.rint(v * 4)
+    A = Csr5.from_csr_device(rows, 30000, *(to_dev(a.astype(np.int32)) for a in (rp, ci)), to_dev(v), sigma=8)
+    x, u = (torch.zeros(n, dtype=torch.float64, device="cuda") for n in (30000, rows))
+    y, z = torch.zeros_like(u), torch.zeros_like(x)
+    A.spmv_transpose(u, z)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        A.spmv(x, y)
+        A.spmv_transpose(u, z)
+    row = np.repeat(np.arange(rows), np.diff(rp.astype(np.int64)))
+    for _ in range(3):
+        xh, uh = rng.integers(-8, 9, 30000).astype(float), rng.integers(-8, 9, rows).astype(float)
+        x.copy_(to_dev(xh))
+        u.copy_(to_dev(uh))
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(y.cpu().numpy(), np.bincount(row, weights=v * xh[ci], minlength=rows))
+        np.testing.assert_array_equal(z.cpu().numpy(), np.bincount(ci, weights=v * uh[row], minlength=30000))
