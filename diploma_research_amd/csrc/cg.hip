@@ -470,12 +470,14 @@ hipError_t plain_product(dim_csr5* A, int k, const double* x, double* y, size_t 
 ResidentPlan resident_plan(const dim_csr5* A, int k, bool mixed) {
     if (!A->dia.nd || (mixed && !A->dia.v32))
         return {};
+    // (a batch of one system keeps its diagonals in the batch's table)
+    const int32_t* off = A->dia.sys_off ? A->sys_off.data() : A->dia.off;
     std::vector<ResidentJob> jobs(static_cast<size_t>(k));
     for (int j = 0; j < k; ++j) {
         jobs[j].row0 = 0;
         jobs[j].rows = A->f.rows;
         jobs[j].vec0 = static_cast<uint64_t>(j) * A->f.rows;
-        std::copy(std::begin(A->dia.off), std::end(A->dia.off), jobs[j].off);
+        std::copy(off, off + kDiaMax, jobs[j].off);
     }
     return plan_resident(std::move(jobs), A->dia.nd, mixed ? sizeof(float) : sizeof(double));
 }
