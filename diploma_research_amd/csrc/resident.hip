@@ -443,7 +443,9 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
                 const V rj = r[j] - alpha * q[j];
                 r[j] = rj;
                 acc += static_cast<double>(rj) * static_cast<double>(rj);
-                if (team.tn > 1 && l < rows && (FAR || l < H || l + H >= rows)) {
+                // (far diagonals are read from memory within a workgroup's
+                // own rows too: a team may be one workgroup)
+                if (l < rows && (FAR || (team.tn > 1 && (l < H || l + H >= rows)))) {
                     if constexpr (WIDE)
                         store_chip(R + first_row + l, rj);
                     else

@@ -26,3 +26,36 @@ def test_batch_of_one_system_as_a_matrix(cuda, grid, precision):
         oc = M.cg(B[:, j].copy(), rtol=1e-10, maxit=2000)
         assert rj.converged and rj.relres_true <= 1.01e-10
         np.testing.assert_allclose(xj.cpu().numpy(), oc["x"], rtol=1e-6, atol=1e-7)
+
+
+# Three diagonals, FP64: a workgroup takes up to 8192 rows, and its window has
+# room for a halo of 1408 entries.
+@pytest.mark.parametrize("rows,off", [(6000, 1500), (8192, 1408), (8192, 1409), (8128, 1600)])
+def test_far_diagonals_of_one_workgroup(cuda, rows, off):
+    """So many systems that most teams are one workgroup, with diagonals that
+    reach past its window but not past its rows: every system's solution."""
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    S = 200
+    rng = np.random.default_rng(rows + off)
+    r = np.arange(rows)
+    at = np.stack([r - off, r, r + off], 1)
+    held = (at >= 0) & (at < rows)
+    rp = np.concatenate([[0], np.cumsum(held.sum(1))]).astype(np.uint32)
+    ci = at[held].astype(np.uint32)
+    systems, xs, bs = [], [], []
+    for _ in range(S):
+        # symmetric: the coupling of rows i and i + off is w[i]; diagonally dominant
+        w = rng.uniform(0.5, 1.0, rows)
+        vals = np.stack([-np.roll(w, off), np.full(rows, 2.5), -w], 1)
+        v = vals[held]
+        x = rng.uniform(-1, 1, rows)
+        systems.append((rows, rp, ci, v))
+        xs.append(x)
+        bs.append(O.csr_spmv(rp, ci, v, x))
+    A = Csr5.from_csr_batched(systems, sigma=5)
+    X, res = conjugate_gradient_batched(A, to_dev(np.concatenate(bs)), rtol=1e-12, max_iters=300)
+    assert all(q.converged and q.relres_true <= 1.01e-12 for q in res)
+    # ||A^-1|| <= 2 and ||A|| <= 4.5: the error is at most 9 times the residual's share
+    x = np.concatenate(xs)
+    assert np.linalg.norm(X.cpu().numpy() - x) <= 1e-11 * np.linalg.norm(x)
