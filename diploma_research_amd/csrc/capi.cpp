@@ -576,6 +576,14 @@ using namespace dimgpu;
 
 extern "C" {
 
+uint32_t dim_test_resident(dim_csr5* A, uint32_t fault, uint32_t from) {
+    const uint32_t ran = A->resident.ran;
+    A->resident = ResidentTrial{};
+    A->resident.fault = fault;
+    A->resident.from = from;
+    return ran;
+}
+
 const char* dim_last_error(void) { return g_last_error.c_str(); }
 
 const char* dim_status_string(dim_status s) {

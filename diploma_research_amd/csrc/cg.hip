@@ -760,13 +760,14 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         rs.max_iters = static_cast<int>(o.max_iters);
         rs.hist = hist;
         rs.hist_cap = hist_cap;
+        const ResidentWaits waits = A->resident.next();
         std::lock_guard<std::mutex> guard(resident_mutex()); // (the stream is idle here)
         DIM_HIP_TRY(launch_resident(plan, mixed, mixed ? static_cast<const void*>(A->dia.v32) : A->dia.v64, A->dia.ld,
                                     mixed ? static_cast<void*>(x32) : x, mixed ? static_cast<void*>(r32) : r64,
-                                    mixed ? static_cast<void*>(p32) : p64, rs, w.res, upload_plan, stream));
-        upload_plan = false;
+                                    mixed ? static_cast<void*>(p32) : p64, rs, waits, w.res, upload_plan, stream));
+        upload_plan = waits.absent;
         if (cc)
-            cc->plan_uploaded = true;
+            cc->plan_uploaded = !upload_plan;
         int code = 0;
         DIM_HIP_TRY(resident_abort(w.res, &code, stream));
         DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
@@ -775,6 +776,7 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
             resident = false;
             return capture();
         }
+        A->resident.ran += !code;
         if (code)
             return fail(DIM_HIP_ERROR, "CG: a wait between the resident solver's workgroups timed out");
         hs->iterations = 0;

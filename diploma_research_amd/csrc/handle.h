@@ -5,6 +5,7 @@
 #include "dia.h"
 #include "dim_internal.h"
 #include "kernels.h"
+#include "resident.h"
 #include "window.h"
 #include "../../include/dim_gpu.h"
 
@@ -65,6 +66,7 @@ struct dim_csr5 {
     dimgpu::DiaForm dia;        // stencil matrices: the values by diagonal (dia.h)
     dimgpu::WindowPlan win;     // matrices within a band (window.h)
     dimgpu::TransposePlan tplan; // made with the first transposed product
+    dimgpu::ResidentTrial resident;
     // Column slices for plain products (capi.cpp): xs is the matrix whose
     // rows are the (column slice s, row i) pairs that hold elements, in the
     // order of s*rows + i. That stacked handle also owns the partial products
@@ -261,3 +263,9 @@ hipError_t launch_dia_fill(const dim_csr5* h, hipStream_t stream);
 hipError_t alloc_diagonals(dim_csr5* h, uint32_t nd, size_t meta, DiaForm& D);
 
 } // namespace dimgpu
+
+// For the tests, and so in no public header: how many resident launches of the
+// handle's solves iterated since the last call; from the next launch but `from`
+// on they fail as `fault` (ResidentTrial::Fault) says. The kernels end by
+// themselves in every case.
+extern "C" uint32_t dim_test_resident(dim_csr5* A, uint32_t fault, uint32_t from);

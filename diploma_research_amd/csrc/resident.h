@@ -48,6 +48,36 @@ constexpr uint32_t kResidentXcds = 8;
 constexpr uint32_t kResidentCus = 32; // workgroups (one per CU) of an XCD
 constexpr uint32_t kResidentRows = 1u << 21; // the largest system: 8192 rows per CU
 
+// How long the workgroups of a launch wait for one another.
+struct ResidentWaits {
+    uint32_t need = kResidentXcds * kResidentCus; // workgroups that must be running
+    double seat_seconds = 1.0;  // for all of them to be running
+    double wait_seconds = 10.0; // for a sum of a meeting (they take microseconds)
+    bool absent = false; // for tests: one workgroup of a team stays away from its meetings
+};
+
+// The tests' hold on a handle's resident launches (dim_test_resident): the
+// launches from number `from` on fail as `fault` says.
+struct ResidentTrial {
+    enum Fault : uint32_t { kNone, kNeverSeated, kWaitsFail };
+    uint32_t fault = kNone, from = 0;
+    uint32_t launches = 0; // since it was set
+    uint32_t ran = 0;      // of those, launches that iterated
+
+    ResidentWaits next() {
+        ResidentWaits w;
+        if (launches++ >= from) {
+            if (fault == kNeverSeated)
+                ++w.need; // a workgroup more than there are
+            if (fault == kWaitsFail) {
+                w.absent = true;
+                w.wait_seconds = 1e-3;
+            }
+        }
+        return w;
+    }
+};
+
 // How a set of systems is shared out.
 struct ResidentPlan {
     bool ok = false;
@@ -77,11 +107,13 @@ size_t resident_bytes(const ResidentPlan& p);
 
 // Runs the iterations of every job until it stops or pauses. work:
 // resident_bytes(p) bytes on a 256-byte boundary; upload: copy the plan into it
-// first (a plan already there may be reused). *abort (in work) is set when the
+// first (a plan already there may be reused; one with an absent workgroup is
+// always copied and none to be reused). *abort (in work) is set when the
 // workgroups could not be seated or a wait timed out; resident_abort() reads
 // it back after the launch.
 hipError_t launch_resident(const ResidentPlan& p, bool f32, const void* vals, uint64_t ld, void* x, void* r, void* p_vec,
-                           const ResidentState& st, void* work, bool upload, hipStream_t stream);
+                           const ResidentState& st, const ResidentWaits& waits, void* work, bool upload,
+                           hipStream_t stream);
 constexpr int kResidentTimeout = 1; // a wait between workgroups passed its limit
 constexpr int kResidentSeats = 2;   // not all workgroups running, or not 32 to an XCD; nothing was touched
 hipError_t resident_abort(const void* work, int* code, hipStream_t stream);

@@ -103,6 +103,7 @@ struct Args {
     Meeting* meet;
     uint64_t limit;      // wall-clock ticks a wait may take
     uint64_t seat_limit; // and the wait for all workgroups to be running
+    uint32_t need;       // how many that are
 };
 
 // What workgroups exchange: a load does not take a line that L1 kept from
@@ -194,8 +195,14 @@ __device__ bool meet(Meeting* m, Team& t, uint64_t limit, double v, double* sum)
                 if (lane > 0 && lane < static_cast<int>(kResidentCus))
                     ok = await_slot(local + lane, m, limit, &u);
                 const double x = wave_total(u);
-                if (lane == 0)
+                // (without one of its parts there is no sum: the word that
+                // ends the other workgroups' waits instead)
+                if (__ballot(!ok)) {
+                    if (lane == 0)
+                        store_chip(&m->abort[0], kResidentTimeout);
+                } else if (lane == 0) {
                     store_chip(&global[t.xcd][0], isnan(x) ? __longlong_as_double(0x7ff8000000000000ll) : x);
+                }
             } else if (lane == 0) {
                 store_xcd(local + t.rank, b);
             }
@@ -221,11 +228,12 @@ __device__ bool meet(Meeting* m, Team& t, uint64_t limit, double v, double* sum)
             if (lane == 0)
                 store_xcd(&m->local[t.xcd][(t.phase + 2u) & 3u][t.rank], __longlong_as_double(kEmpty));
         }
-        if (__ballot(!ok) && lane == 0)
-            store_chip(&m->abort[0], kResidentTimeout);
+        const bool all = __ballot(!ok) == 0ull; // (of all lanes: not below lane 0's branch)
         if (lane == 0) {
+            if (!all)
+                store_chip(&m->abort[0], kResidentTimeout);
             total = b;
-            good = __ballot(!ok) == 0ull;
+            good = all;
         }
     }
     ++t.phase;
@@ -519,7 +527,7 @@ __global__ __launch_bounds__(kThreads) void k_resident(Args<V> a) {
         int state = 0;
         for (;;) {
             const unsigned c = load_shared(&a.meet->total[0]);
-            if (c == gridDim.x)
+            if (c == a.need)
                 break;
             if (c >= kCalledOff) {
                 state = kResidentSeats;
@@ -527,7 +535,7 @@ __global__ __launch_bounds__(kThreads) void k_resident(Args<V> a) {
             }
             if (wall_clock64() - t0 > a.seat_limit) {
                 if (__hip_atomic_fetch_add(&a.meet->total[0], kCalledOff, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT) != gridDim.x)
+                                           __HIP_MEMORY_SCOPE_AGENT) != a.need)
                     state = kResidentSeats;
                 break;
             }
@@ -623,7 +631,7 @@ hipError_t launch_nd(const ResidentPlan& p, const Args<V>& a, hipStream_t s) {
 
 template<typename V>
 hipError_t run(const ResidentPlan& p, const void* vals, uint64_t ld, void* x, void* r, void* pv,
-               const ResidentState& st, char* work, hipStream_t s) {
+               const ResidentState& st, const ResidentWaits& waits, char* work, hipStream_t s) {
     int dev = 0, khz = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess)
@@ -642,9 +650,10 @@ hipError_t run(const ResidentPlan& p, const void* vals, uint64_t ld, void* x, vo
                                                     up256(p.jobs.size() * sizeof(ResidentJob)));
     a.rounds = p.rounds;
     a.st = st;
-    const uint64_t second = static_cast<uint64_t>(std::max(khz, 1)) * 1000ull;
-    a.limit = 10 * second; // a wait takes microseconds
-    a.seat_limit = second;
+    const double second = std::max(khz, 1) * 1e3;
+    a.limit = static_cast<uint64_t>(waits.wait_seconds * second);
+    a.seat_limit = static_cast<uint64_t>(waits.seat_seconds * second);
+    a.need = waits.need;
     hipLaunchKernelGGL(k_clear, dim3(1), dim3(1024), 0, s, a.meet);
     return launch_nd<V>(p, a, s);
 }
@@ -841,22 +850,35 @@ size_t resident_bytes(const ResidentPlan& p) {
 }
 
 hipError_t launch_resident(const ResidentPlan& p, bool f32, const void* vals, uint64_t ld, void* x, void* r, void* p_vec,
-                           const ResidentState& st, void* work, bool upload, hipStream_t stream) {
+                           const ResidentState& st, const ResidentWaits& waits, void* work, bool upload,
+                           hipStream_t stream) {
     if (!p.ok)
         return hipErrorInvalidValue;
     char* w = static_cast<char*>(work);
-    if (upload) {
+    if (upload || waits.absent) {
         const size_t at = up256(sizeof(Meeting));
         hipError_t e = hipMemcpyAsync(w + at, p.jobs.data(), p.jobs.size() * sizeof(ResidentJob),
                                       hipMemcpyHostToDevice, stream);
+        std::vector<ResidentSeat> seats;
+        if (waits.absent) {
+            seats = p.seats;
+            for (ResidentSeat& s : seats)
+                if (s.job != kNoJob && s.tb && s.tb == s.tn - 1) {
+                    s.job = kNoJob;
+                    break;
+                }
+        }
         if (e == hipSuccess)
-            e = hipMemcpyAsync(w + at + up256(p.jobs.size() * sizeof(ResidentJob)), p.seats.data(),
-                               p.seats.size() * sizeof(ResidentSeat), hipMemcpyHostToDevice, stream);
+            e = hipMemcpyAsync(w + at + up256(p.jobs.size() * sizeof(ResidentJob)),
+                               waits.absent ? seats.data() : p.seats.data(), p.seats.size() * sizeof(ResidentSeat),
+                               hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess && waits.absent)
+            e = hipStreamSynchronize(stream);
         if (e != hipSuccess)
             return e;
     }
-    return f32 ? run<float>(p, vals, ld, x, r, p_vec, st, w, stream)
-               : run<double>(p, vals, ld, x, r, p_vec, st, w, stream);
+    return f32 ? run<float>(p, vals, ld, x, r, p_vec, st, waits, w, stream)
+               : run<double>(p, vals, ld, x, r, p_vec, st, waits, w, stream);
 }
 
 hipError_t resident_abort(const void* work, int* code, hipStream_t stream) {

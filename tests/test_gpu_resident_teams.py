@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 from gpu_util import to_dev
-from diploma_research_amd import Csr5, conjugate_gradient, conjugate_gradient_multi, matgen
+from diploma_research_amd import Csr5, DimError, conjugate_gradient, conjugate_gradient_multi, matgen
+from diploma_research_amd import native as N
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -59,3 +60,37 @@ def test_far_diagonals_of_one_workgroup(cuda, rows, off):
     # ||A^-1|| <= 2 and ||A|| <= 4.5: the error is at most 9 times the residual's share
     x = np.concatenate(xs)
     assert np.linalg.norm(X.cpu().numpy() - x) <= 1e-11 * np.linalg.norm(x)
+
+
+# The faults that the tests' hold on a handle can set
+NONE, NEVER_SEATED, WAITS_FAIL = range(3)
+
+
+def _resident(A, fault=NONE, start=0):
+    """Resident launches of A's solves that iterated since the last call;
+    those from the next but `start` on fail."""
+    return N.lib().dim_test_resident(A._h, fault, start)
+
+
+# one team on an XCD; the whole chip
+@pytest.mark.parametrize("grid", [(61, 67), (103, 104, 105)])
+def test_failed_wait_stops_every_workgroup(cuda, grid):
+    """One workgroup stays away from the meetings: the waits for it end by their
+    limit and stop every workgroup, the solve reports it, x keeps what it held,
+    and the next solve is as ever."""
+    import torch
+
+    rp, ci, v = matgen.varcoef(grid, 0.5, seed=9)
+    n = len(rp) - 1
+    b = to_dev(np.random.default_rng(9).uniform(-1, 1, n))
+    A = Csr5.from_csr((n, n, rp, ci, v), sigma=8)
+    x0 = torch.linspace(-1, 1, n, dtype=torch.float64, device="cuda")
+    _resident(A, WAITS_FAIL)
+    x = x0.clone()
+    with pytest.raises(DimError, match="timed out"):
+        conjugate_gradient(A, b, x=x, rtol=1e-10, max_iters=3000)
+    assert torch.equal(x, x0)
+    assert _resident(A) == 0
+    x, r = conjugate_gradient(A, b, x=x, rtol=1e-10, max_iters=3000)
+    assert _resident(A) == 1
+    assert r.converged and r.relres_true <= 1.01e-10
