@@ -38,6 +38,7 @@
 // it, block reduction included): 1.1 us for 2 to 32 workgroups of an XCD, 2.4
 // us for the chip in two levels.
 #include "resident.h"
+#include "seating.h"
 #include "spmv_impl.h"
 
 #include <algorithm>
@@ -78,7 +79,6 @@ constexpr bool far_in_registers(uint32_t nd, uint32_t rpt, size_t vb) {
     const bool res = values_resident(nd, rpt, vb);
     return ((res ? rpt : chunk_rows(rpt)) * nd + (x_in_lds(nd, rpt, vb) ? 4 : 5) * rpt) * vb / 4 <= (res ? 165 : 190);
 }
-constexpr unsigned kCalledOff = 0x10000; // added to the seat count
 constexpr long long kEmpty = -1; // a slot nobody has written: no sum has these bits
 
 // Meeting slots, counters and the abort word, cleared before every launch.
@@ -318,6 +318,10 @@ __device__ bool run_job(const Args<V>& a, uint32_t job, Team& team, V* win) {
     int status = 0;
     bool ok = true;
     for (;;) {
+        // The loop's first line of instructions is a whole one, wherever the code
+        // before it ends (8 FP32-refined columns of 64^3 cells: 10.8 ms, and 11.15
+        // with an end that does not suit).
+        asm volatile(".p2align 6");
         // (opaque, so that the many addresses made from it are made anew in
         // every iteration instead of being kept in registers throughout)
         uint32_t tid = threadIdx.x;
@@ -521,26 +525,24 @@ __global__ __launch_bounds__(kThreads) void k_resident(Args<V> a) {
         __hip_atomic_fetch_add(&a.meet->total[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // All workgroups are running when the count is complete; from then on
         // every wait ends. One that has waited too long for the others (CUs
-        // held by another program) calls the launch off, unless the count is
-        // complete by then: nobody sees a complete count after its addition.
+        // held by another program) calls the launch off.
+        struct {
+            unsigned* p;
+            __device__ unsigned load() { return load_shared(p); }
+            __device__ bool replace(unsigned from, unsigned to) {
+                return __hip_atomic_compare_exchange_strong(p, &from, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } count{&a.meet->total[0]};
         const uint64_t t0 = wall_clock64();
-        int state = 0;
+        Seats seats = Seats::kWaiting;
         for (;;) {
-            const unsigned c = load_shared(&a.meet->total[0]);
-            if (c == a.need)
+            seats = look_at_seats(count, a.need, wall_clock64() - t0 > a.seat_limit);
+            if (seats != Seats::kWaiting)
                 break;
-            if (c >= kCalledOff) {
-                state = kResidentSeats;
-                break;
-            }
-            if (wall_clock64() - t0 > a.seat_limit) {
-                if (__hip_atomic_fetch_add(&a.meet->total[0], kCalledOff, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT) != a.need)
-                    state = kResidentSeats;
-                break;
-            }
             __builtin_amdgcn_s_sleep(1);
         }
+        int state = seats == Seats::kComplete ? 0 : kResidentSeats;
         if (!state)
             for (uint32_t i = 0; i < kResidentXcds; ++i)
                 if (load_shared(&a.meet->seated[i][0]) != kResidentCus)

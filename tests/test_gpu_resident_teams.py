@@ -94,3 +94,28 @@ def test_failed_wait_stops_every_workgroup(cuda, grid):
     x, r = conjugate_gradient(A, b, x=x, rtol=1e-10, max_iters=3000)
     assert _resident(A) == 1
     assert r.converged and r.relres_true <= 1.01e-10
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32-refined"])
+def test_never_seated_takes_the_launch_sequence(cuda, precision):
+    """Workgroups that are not all running call the launch off: the launch
+    sequence solves, single systems and batches alike."""
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    rp, ci, v = matgen.varcoef((40, 41), 0.5, seed=2)
+    n = len(rp) - 1
+    b = np.random.default_rng(2).uniform(-1, 1, n)
+    oc = O.Csr5(n, n, rp, ci, v).cg(b, rtol=1e-10, maxit=2000)
+    A = Csr5.from_csr((n, n, rp, ci, v), sigma=8, keep_f32=True)
+    _resident(A, NEVER_SEATED)
+    x, r = conjugate_gradient(A, to_dev(b), rtol=1e-10, max_iters=2000, precision=precision)
+    assert _resident(A) == 0
+    assert r.converged and r.relres_true <= 1.01e-10
+    np.testing.assert_allclose(x.cpu().numpy(), oc["x"], rtol=1e-6, atol=1e-7)
+    if precision == "f64":
+        S = Csr5.from_csr_batched([(n, rp, ci, v)] * 3, sigma=8)
+        _resident(S, NEVER_SEATED)
+        X, R = conjugate_gradient_batched(S, to_dev(np.tile(b, 3)), rtol=1e-10, max_iters=2000)
+        assert _resident(S) == 0
+        assert all(q.converged for q in R)
+        np.testing.assert_allclose(X.cpu().numpy(), np.tile(oc["x"], 3), rtol=1e-7, atol=1e-8)
