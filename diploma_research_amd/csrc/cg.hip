@@ -744,6 +744,26 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
                        o.rtol, delta * delta, hist);
     DIM_HIP_TRY(hipGetLastError());
 
+    // From the resident solver to the launch sequence, whose columns share one
+    // count: it goes on from the furthest column that has not stopped, so that
+    // none passes max_iters, and the results add what each column has behind.
+    int left_at = 0;                   // the shared count at that point
+    std::array<int, kMaxK> left_run{}; // and the column's own, -1 if it had stopped
+    auto leave_resident = [&]() -> dim_status {
+        resident = false;
+        for (int j = 0; j < k; ++j) {
+            left_run[j] = hs->col_done[j] ? -1 : hs->col_run[j];
+            left_at = std::max(left_at, left_run[j]);
+        }
+        if (left_at > 0) {
+            hs->iterations = left_at;
+            hs->done = left_at >= static_cast<int>(o.max_iters) ? 3 : 0;
+            DIM_HIP_TRY(hipMemcpyAsync(&st->iterations, &hs->iterations, sizeof(int), hipMemcpyHostToDevice, stream));
+            DIM_HIP_TRY(hipMemcpyAsync(&st->done, &hs->done, sizeof(int), hipMemcpyHostToDevice, stream));
+        }
+        return capture();
+    };
+
     // Every column's iterations on the resident solver, until it stops (or,
     // FP32-refined, its residual is to be replaced). A launch whose workgroups
     // are not seated as the plan assumes says so before it touches anything;
@@ -772,10 +792,8 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         DIM_HIP_TRY(resident_abort(w.res, &code, stream));
         DIM_HIP_TRY(hipMemcpyAsync(hs, st, sizeof(CgState), hipMemcpyDeviceToHost, stream));
         DIM_HIP_TRY(hipStreamSynchronize(stream));
-        if (code == kResidentSeats) {
-            resident = false;
-            return capture();
-        }
+        if (code == kResidentSeats)
+            return leave_resident();
         A->resident.ran += !code;
         if (code)
             return fail(DIM_HIP_ERROR, "CG: a wait between the resident solver's workgroups timed out");
@@ -881,6 +899,8 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         dim_cg_result& R = res[j];
         R.converged = S.col_done[j] == 1;
         R.iterations = static_cast<uint32_t>(S.col_done[j] ? S.col_iters[j] : resident ? S.col_run[j] : S.iterations);
+        if (left_at > 0 && left_run[j] >= 0)
+            R.iterations += left_run[j] - left_at;
         R.relres = std::sqrt(mixed ? S.rr_true[j] : S.rr[j]) / scale;
         R.relres_true = std::sqrt(tr) / scale;
         R.refinements = refinements;

@@ -119,3 +119,42 @@ def test_never_seated_takes_the_launch_sequence(cuda, precision):
         assert _resident(S) == 0
         assert all(q.converged for q in R)
         np.testing.assert_allclose(X.cpu().numpy(), np.tile(oc["x"], 3), rtol=1e-7, atol=1e-8)
+
+
+@pytest.mark.parametrize("k", [1, 3])
+def test_called_off_after_a_refinement(cuda, k):
+    """The launch sequence takes over where the resident launches end in the
+    middle of an FP32-refined solve: the columns' counts, the history and the
+    cap are those of one solve."""
+    rp, ci, v = matgen.varcoef((40, 41), 0.5, seed=6)
+    n = len(rp) - 1
+    B = np.random.default_rng(6).uniform(-1, 1, (n, k)) * 10.0 ** -np.arange(k)
+    A = Csr5.from_csr((n, n, rp, ci, v), sigma=8, keep_f32=True)
+
+    def run(max_iters, **kw):
+        if k == 1:
+            x, r = conjugate_gradient(A, to_dev(B[:, 0].copy()), rtol=1e-10, max_iters=max_iters, **kw)
+            return x[:, None], [r]
+        return conjugate_gradient_multi(A, to_dev(B), rtol=1e-10, max_iters=max_iters, **kw)
+
+    hist = {"history": True} if k == 1 else {}
+    X0, R0 = run(2000, precision="f32-refined", **hist)
+    assert _resident(A, NEVER_SEATED, 1) > 1
+    X1, R1 = run(2000, precision="f32-refined", **hist)
+    assert _resident(A, NEVER_SEATED, 1) == 1
+    for j in range(k):
+        assert R1[j].converged and R1[j].relres_true <= 1.01e-10
+        # the forms round differently, which moves a stop by a few steps
+        assert abs(R1[j].iterations - R0[j].iterations) <= 0.03 * R0[j].iterations + 3
+        oc = O.Csr5(n, n, rp, ci, v).cg(B[:, j].copy(), rtol=1e-10, maxit=2000)
+        np.testing.assert_allclose(X1[:, j].cpu().numpy(), oc["x"], rtol=1e-6, atol=1e-7)
+    if k == 1:
+        h0, h1 = np.asarray(R0[0].history), np.asarray(R1[0].history)
+        m = min(R0[0].iterations, R1[0].iterations) - 5
+        assert (h1[:m] > 0).all()
+        # both follow one residual, which falls by ten orders of magnitude
+        assert np.abs(np.log10(h1[:m]) - np.log10(h0[:m])).max() < 1.0
+    cap = R0[0].iterations * 2 // 3
+    _, R2 = run(cap, precision="f32-refined")
+    assert _resident(A) == 1
+    assert max(r.iterations for r in R2) == cap and not R2[0].converged
