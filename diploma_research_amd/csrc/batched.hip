@@ -1135,19 +1135,21 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
         rs.iters = sa.sys_iters;
         rs.run = sa.run;
         rs.max_iters = static_cast<int>(o.max_iters);
-        const ResidentWaits waits = A->resident.next();
         DIM_HIP_TRY(hipStreamSynchronize(stream));
-        std::lock_guard<std::mutex> guard(resident_mutex());
-        DIM_HIP_TRY(launch_resident(bc->plan, false, A->dia.v64, A->dia.ld, x, r, p, rs, waits, bc->res,
-                                    !bc->plan_uploaded, stream));
-        bc->plan_uploaded = !waits.absent;
-        int code = 0;
-        DIM_HIP_TRY(resident_abort(bc->res, &code, stream));
-        DIM_HIP_TRY(hipStreamSynchronize(stream));
-        if (code && code != kResidentSeats)
-            return fail(DIM_HIP_ERROR, "batched CG: a wait between the resident solver's workgroups timed out");
-        iterated = !code;
-        A->resident.ran += iterated;
+        const std::unique_lock<std::timed_mutex> guard = resident_lock();
+        if (guard) {
+            const ResidentWaits waits = A->resident.next();
+            DIM_HIP_TRY(launch_resident(bc->plan, false, A->dia.v64, A->dia.ld, x, r, p, rs, waits, bc->res,
+                                        !bc->plan_uploaded, stream));
+            bc->plan_uploaded = !waits.absent;
+            int code = 0;
+            DIM_HIP_TRY(resident_abort(bc->res, &code, stream));
+            DIM_HIP_TRY(hipStreamSynchronize(stream));
+            if (code && code != kResidentSeats)
+                return fail(DIM_HIP_ERROR, "batched CG: a wait between the resident solver's workgroups timed out");
+            iterated = !code;
+            A->resident.ran += iterated;
+        }
         hs->iterations = static_cast<int>(o.max_iters); // of the systems that have not stopped
     }
     if (iterated) {

@@ -780,8 +780,10 @@ dim_status solve(dim_csr5* A, int k, const double* b_in, double* x_out, const di
         rs.max_iters = static_cast<int>(o.max_iters);
         rs.hist = hist;
         rs.hist_cap = hist_cap;
+        const std::unique_lock<std::timed_mutex> guard = resident_lock(); // (the stream is idle here)
+        if (!guard)
+            return leave_resident();
         const ResidentWaits waits = A->resident.next();
-        std::lock_guard<std::mutex> guard(resident_mutex()); // (the stream is idle here)
         DIM_HIP_TRY(launch_resident(plan, mixed, mixed ? static_cast<const void*>(A->dia.v32) : A->dia.v64, A->dia.ld,
                                     mixed ? static_cast<void*>(x32) : x, mixed ? static_cast<void*>(r32) : r64,
                                     mixed ? static_cast<void*>(p32) : p64, rs, waits, w.res, upload_plan, stream));

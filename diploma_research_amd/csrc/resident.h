@@ -48,10 +48,17 @@ constexpr uint32_t kResidentXcds = 8;
 constexpr uint32_t kResidentCus = 32; // workgroups (one per CU) of an XCD
 constexpr uint32_t kResidentRows = 1u << 21; // the largest system: 8192 rows per CU
 
+// How long a solve waits for the chip, first for another solve of the process
+// and then for its own workgroups to be running (CUs held by other streams or
+// processes), before it takes the launch sequence. Between the two a small
+// system loses 3 to 14 ms (256^2 cells: 2.9 ms here, 16.7 there), so a longer
+// wait costs more than it can save.
+constexpr double kResidentPatience = 0.01;
+
 // How long the workgroups of a launch wait for one another.
 struct ResidentWaits {
     uint32_t need = kResidentXcds * kResidentCus; // workgroups that must be running
-    double seat_seconds = 1.0;  // for all of them to be running
+    double seat_seconds = kResidentPatience; // for all of them to be running
     double wait_seconds = 10.0; // for a sum of a meeting (they take microseconds)
     bool absent = false; // for tests: one workgroup of a team stays away from its meetings
 };
@@ -95,8 +102,9 @@ bool resident_device();
 
 // Held (per device) from launch_resident() until the launch has ended. The
 // stream must be idle when it is taken, so that nothing a holder waits for can
-// depend on another thread's solve.
-std::mutex& resident_mutex();
+// depend on another thread's solve. Empty when the other solves take longer
+// than kResidentPatience.
+std::unique_lock<std::timed_mutex> resident_lock();
 
 // The plan for `jobs` (row0, rows, vec0 and off filled in) with nd diagonals
 // and values of vb bytes; !ok when they do not fit.

@@ -30,9 +30,10 @@
 // The launch is an ordinary one: a cooperative launch takes a resource that
 // only one process on the GPU can hold. Its workgroups first wait until all of
 // them are running, and call the launch off, with nothing touched, if that does
-// not come about; the caller then solves by launch sequence. Solves of one
-// process do not run side by side (each would hold CUs that the other waits
-// for).
+// not come about soon; the caller then solves by launch sequence. Two resident
+// solves of one process do not run side by side (each would hold CUs that the
+// other waits for): one that would have to wait long for another takes the
+// launch sequence too.
 //
 // Measured (one double per workgroup summed over the team and known to all of
 // it, block reduction included): 1.1 us for 2 to 32 workgroups of an XCD, 2.4
@@ -42,6 +43,7 @@
 #include "spmv_impl.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 
 namespace dimgpu {
@@ -662,11 +664,11 @@ hipError_t run(const ResidentPlan& p, const void* vals, uint64_t ld, void* x, vo
 
 } // namespace
 
-std::mutex& resident_mutex() {
-    static std::mutex per_device[64];
+std::unique_lock<std::timed_mutex> resident_lock() {
+    static std::timed_mutex per_device[64];
     int dev = 0;
     (void)hipGetDevice(&dev);
-    return per_device[dev & 63];
+    return std::unique_lock<std::timed_mutex>(per_device[dev & 63], std::chrono::duration<double>(kResidentPatience));
 }
 
 bool resident_device() {

@@ -158,3 +158,72 @@ def test_called_off_after_a_refinement(cuda, k):
     _, R2 = run(cap, precision="f32-refined")
     assert _resident(A) == 1
     assert max(r.iterations for r in R2) == cap and not R2[0].converged
+
+
+def test_a_held_chip_costs_a_small_solve_little(cuda):
+    """CUs that do not come free are waited for a hundredth of a second."""
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    rp, ci, v = matgen.varcoef((24, 25), 0.5, seed=3)
+    n = len(rp) - 1
+    b = to_dev(np.random.default_rng(3).uniform(-1, 1, n))
+    A = Csr5.from_csr((n, n, rp, ci, v), sigma=8)
+    S = Csr5.from_csr_batched([(n, rp, ci, v)], sigma=8)
+    for _ in range(2):  # (the first solves also load the kernels)
+        _resident(A, NEVER_SEATED)
+        _resident(S, NEVER_SEATED)
+        _, r = conjugate_gradient(A, b, rtol=1e-10)
+        _, (q,) = conjugate_gradient_batched(S, b, rtol=1e-10)
+    assert r.converged and r.seconds < 0.3
+    assert q.converged and q.seconds < 0.3
+
+
+def test_solves_of_other_handles_are_not_held_up(cuda):
+    """A small solve beside another thread's long one ends before it."""
+    import threading
+    import time
+
+    import torch
+
+    # about 2 us an iteration, and far more of them than the tolerance needs
+    rp, ci, v = matgen.varcoef((520, 520), 2.0, seed=1)
+    n = len(rp) - 1
+    long = Csr5.from_csr((n, n, rp, ci, v), sigma=8)
+    b = to_dev(np.random.default_rng(1).uniform(-1, 1, n))
+    rs, cs, vs = matgen.varcoef((40, 41), 0.5, seed=2)
+    m = len(rs) - 1
+    short = Csr5.from_csr((m, m, rs, cs, vs), sigma=8)
+    bs = np.random.default_rng(2).uniform(-1, 1, m)
+    conjugate_gradient(short, to_dev(bs), rtol=1e-10)
+    conjugate_gradient(long, b, rtol=1e-1, max_iters=5)
+    s_long, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(8)]
+    bd, marks = to_dev(bs), [torch.zeros(8, device="cuda") for _ in others]
+    torch.cuda.synchronize()
+    ended = {}
+
+    def solve_long():
+        conjugate_gradient(long, b, x=torch.zeros_like(b), rtol=1e-200, max_iters=100000, stream=s_long)
+        ended["long"] = time.perf_counter()
+
+    t = threading.Thread(target=solve_long)
+    x0 = torch.zeros_like(bd)
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    t.start()
+    # a stream that does not share the long solve's hardware queue
+    events = [torch.cuda.Event() for _ in others]
+    for q, e, mark in zip(others, events, marks):
+        with torch.cuda.stream(q):
+            mark.add_(1)
+        e.record(q)
+    time.sleep(0.05)
+    free = [q for q, e in zip(others, events) if e.query()]
+    assert free and t.is_alive()
+    x, r = conjugate_gradient(short, bd, x=x0, rtol=1e-10, stream=free[0])
+    ended["short"] = time.perf_counter()
+    t.join()
+    assert r.converged and r.relres_true <= 1.01e-10
+    assert ended["long"] - t0 > 0.3, "the long solve is not long"
+    assert ended["short"] < ended["long"]
+    oc = O.Csr5(m, m, rs, cs, vs).cg(bs, rtol=1e-10, maxit=2000)
+    np.testing.assert_allclose(x.cpu().numpy(), oc["x"], rtol=1e-7, atol=1e-8)
