@@ -1073,9 +1073,16 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
     const bool transpose = (o.flags & DIM_CG_TRANSPOSE) != 0;
     const bool codes = A->f.col_code != nullptr;
     const bool persistent = (o.flags & DIM_CG_PERSISTENT) != 0;
-    const int occ = persistent && !A->dia.nd ? persistent_occupancy(A->f.sigma, codes) : 1;
-    if (occ < 1)
-        return fail(DIM_UNSUPPORTED, "batched CG: the persistent kernel cannot be resident for this format");
+    // the cooperative kernel needs its blocks resident; batches kept by diagonals
+    // come to it only when the resident workgroups cannot be seated
+    const auto persistent_fits = [&]() -> dim_status {
+        if (persistent_occupancy(A->f.sigma, codes) < 1)
+            return fail(DIM_UNSUPPORTED, "batched CG: the persistent kernel cannot be resident for this format");
+        return DIM_SUCCESS;
+    };
+    if (persistent && !A->dia.nd)
+        if (dim_status e = persistent_fits())
+            return e;
     const size_t n = A->f.rows;
     const uint32_t check = o.check_every ? o.check_every : 16;
     // the handle's buffers (kept from its first solve), or this call's
@@ -1155,6 +1162,9 @@ dim_status solve_batched(dim_csr5* A, const double* b, double* x, const dim_cg_o
     if (iterated) {
         // (done)
     } else if (persistent) {
+        if (A->dia.nd)
+            if (dim_status e = persistent_fits())
+                return e;
         // one cooperative launch runs every iteration; its vector work items
         // are the launch sequence's blocks (same rows, same reduction order)
         double *rr_part = nullptr, *dot_chunk = nullptr;

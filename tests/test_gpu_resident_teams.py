@@ -227,3 +227,32 @@ def test_solves_of_other_handles_are_not_held_up(cuda):
     assert ended["short"] < ended["long"]
     oc = O.Csr5(m, m, rs, cs, vs).cg(bs, rtol=1e-10, maxit=2000)
     np.testing.assert_allclose(x.cpu().numpy(), oc["x"], rtol=1e-7, atol=1e-8)
+
+
+@pytest.mark.parametrize("sigma", [5, 16])
+def test_called_off_batches_take_the_form_asked_for(cuda, sigma):
+    """Where the resident workgroups are not seated, a batch kept by diagonals
+    is solved by the launch sequence or, with persistent=True, by the
+    cooperative kernel: the same bits."""
+    import torch
+
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    systems = []
+    for i, side in enumerate([11, 37, 5, 60, 23, 48]):
+        rp, ci, v = matgen.varcoef((side, side), 0.5, seed=i)
+        systems.append((side * side, rp, ci, v))
+    A = Csr5.from_csr_batched(systems, sigma=sigma)
+    b = to_dev(np.random.default_rng(0).uniform(-1, 1, sum(n for n, *_ in systems)))
+    got = []
+    for persistent in (False, True, True):
+        _resident(A, NEVER_SEATED)
+        X, R = conjugate_gradient_batched(A, b, rtol=1e-10, max_iters=3000, persistent=persistent)
+        assert all(r.converged and r.relres_true <= 1.01e-10 for r in R)
+        got.append((X, [r.iterations for r in R]))
+    for X, its in got[1:]:
+        assert torch.equal(X, got[0][0]) and its == got[0][1]
+    assert _resident(A) == 0
+    Xr, _ = conjugate_gradient_batched(A, b, rtol=1e-10, max_iters=3000)
+    assert _resident(A) == 1
+    np.testing.assert_allclose(Xr.cpu().numpy(), got[0][0].cpu().numpy(), rtol=1e-7, atol=1e-8)
