@@ -707,6 +707,17 @@ uint32_t fit_job(ResidentJob& j, uint32_t nd, uint32_t tn, uint32_t rpt, size_t 
 
 } // namespace
 
+// When systems take turns, one after another on an XCD's 32 workgroups, an
+// iteration of them all takes about the first sum on the XCD with the most,
+// and in the launch sequence, all systems side by side, the second. The plan is
+// refused where the second is smaller. Measured (5 diagonals, FP64, microseconds
+// an iteration, turns and launch sequence): 272 systems of 500 rows 97 and 34;
+// 192 of 4200 rows 65 and 51, 1024 of them 347 and 194; 96 of 16250 rows 36 and
+// 56; 96 of 62400 rows 43 and 154. The sums are within a third of these and on
+// the right side in all of 35 such pairs.
+constexpr double kTurnMicros = 2.7, kTurnRowMicros = 1.5e-5;
+constexpr double kSequenceMicros = 11.0, kSequenceJobMicros = 0.04, kSequenceRowMicros = 2.75e-5;
+
 ResidentPlan plan_resident(std::vector<ResidentJob> jobs, uint32_t nd, size_t vb) {
     ResidentPlan p;
     p.nd = nd;
@@ -810,9 +821,20 @@ ResidentPlan plan_resident(std::vector<ResidentJob> jobs, uint32_t nd, size_t vb
         }
     }
     p.rounds = 1;
+    double turns_us = 0.0; // an iteration of everything on the XCD with the longest turns
     for (uint32_t x = 0; x < kResidentXcds; ++x)
-        if (shares[x].turns)
+        if (shares[x].turns) {
             p.rounds = std::max(p.rounds, static_cast<uint32_t>(of[x].size()));
+            double us = 0.0;
+            for (uint32_t i : of[x])
+                us += kTurnMicros + kTurnRowMicros * jobs[i].rows;
+            turns_us = std::max(turns_us, us);
+        }
+    uint64_t all_rows = 0;
+    for (const ResidentJob& j : jobs)
+        all_rows += j.rows;
+    if (turns_us > kSequenceMicros + kSequenceJobMicros * jobs.size() + kSequenceRowMicros * all_rows)
+        return p;
     p.seats.assign(size_t{p.rounds} * kSeatsAll, ResidentSeat{kNoJob, 0, 0, 0});
     // rows per thread first: the window's room for a halo depends on it
     for (uint32_t x = 0; x < kResidentXcds; ++x)

@@ -256,3 +256,28 @@ def test_called_off_batches_take_the_form_asked_for(cuda, sigma):
     Xr, _ = conjugate_gradient_batched(A, b, rtol=1e-10, max_iters=3000)
     assert _resident(A) == 1
     np.testing.assert_allclose(Xr.cpu().numpy(), got[0][0].cpu().numpy(), rtol=1e-7, atol=1e-8)
+
+
+# many small systems, which the launch sequence iterates side by side, and a few
+# that fill an XCD each
+@pytest.mark.parametrize("shape,systems,resident", [((20, 25), 256, 1), ((20, 25), 300, 0), ((60, 70), 200, 0),
+                                                    ((300, 310), 20, 1)])
+def test_batches_that_would_take_too_many_turns(cuda, shape, systems, resident):
+    from diploma_research_amd.csr5 import conjugate_gradient_batched
+
+    rp, ci, v = matgen.varcoef(shape, 0.5, seed=systems)
+    n = len(rp) - 1
+    A = Csr5.from_csr_batched([(n, rp, ci, v)] * systems, sigma=5)
+    x = np.random.default_rng(systems).uniform(-1, 1, (systems, n))
+    some = sorted({0, 1, systems // 2, systems - 1})
+    b = np.zeros((systems, n))
+    for i in range(systems):
+        b[i] = O.csr_spmv(rp, ci, v, x[i])
+    _resident(A)
+    X, R = conjugate_gradient_batched(A, to_dev(b.ravel()), rtol=1e-10, max_iters=5000)
+    assert _resident(A) == resident
+    assert all(r.converged and r.relres_true <= 1.01e-10 for r in R)
+    X = X.cpu().numpy().reshape(systems, n)
+    for i in some:
+        oc = O.Csr5(n, n, rp, ci, v).cg(b[i], rtol=1e-10, maxit=5000)
+        np.testing.assert_allclose(X[i], oc["x"], rtol=1e-6, atol=1e-7)
