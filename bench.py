@@ -112,13 +112,14 @@ def stream_read_ceiling(gib=4, reps=5):
     return round(best, 1)
 
 
-def by_diagonals(sigma, codes):
-    """Whether products of the 7-point operator take the diagonal form's kernel
-    (no row of 7 spans three lanes of a tile)."""
-    return codes and sigma >= 6
+def by_diagonals(sigma, plain_columns=False):
+    """Whether products of the 7-point operator take the diagonal form's kernel:
+    unless told to keep plain columns, where a row of 7 is no longer than sigma
+    (the library's rule for rows within two lanes of a tile)."""
+    return not plain_columns and sigma >= 7
 
 
-def traffic_for(sigma, codes):
+def traffic_for(sigma, codes, plain_columns=False):
     """HBM bytes per launch of the headline kernel at `sigma` from the
     committed rocprofv3 FETCH_SIZE / WRITE_SIZE runs (profiles/)."""
     tfile = os.path.join(ROOT, "profiles", "spmv_tiles_f64_poisson128_traffic.json")
@@ -126,7 +127,7 @@ def traffic_for(sigma, codes):
         return None
     with open(tfile) as f:
         t = json.load(f)
-    key = "dia" if by_diagonals(sigma, codes) else f"{sigma}{'c' if codes else ''}"
+    key = "dia" if by_diagonals(sigma, plain_columns) else f"{sigma}{'c' if codes else ''}"
     entry = t.get("by_kernel", {}).get(key) or t.get("by_sigma", {}).get(str(sigma))
     return entry.get("hbm_bytes_per_launch") if entry else None
 
@@ -636,7 +637,7 @@ def main():
     ms_plain = time_spmv(pmats, pxs, pys, a.steps, a.warmup)
     plain = {"sigma": P0.sigma, "ms": round(ms_plain, 5), "GB/s": round(bytes_step / ms_plain / 1e6, 2),
              "frac_hbm_peak": round(bytes_step / ms_plain / 1e6 / HBM_PEAK_GBS, 4),
-             "traffic": traffic_for(P0.sigma, False)}
+             "traffic": traffic_for(P0.sigma, False, plain_columns=True)}
     del pmats, pxs, pys, P0
     ceiling = stream_read_ceiling()
     traffic = traffic_for(sigma, codes)
@@ -738,11 +739,14 @@ def main():
                    "sigma": sigma, "omega": 64, "bytes_per_step": bytes_step, "column_codes": codes,
                    "frac_hbm_peak": round(gbs / HBM_PEAK_GBS, 4), "warm_GB/s": gbs_warm,
                    "plain_columns": plain, "host_pointers": host_ptrs, "stream_read_ceiling_GB/s": ceiling,
-                   "frac_stream_ceiling": round(gbs / ceiling, 4) if ceiling else None,
+                   # of the bytes that pass, where they are known (the diagonal form reads no columns)
+                   "frac_stream_ceiling": round((traffic or bytes_step) / ms / 1e6 / ceiling, 4) if ceiling else None,
                    "parity_rel_err_vs_cpu_baseline": parity},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_dia_spmv<double,7,true>" if by_diagonals(sigma, codes) else
+                     "traffic_GB/s": round(traffic / kernel_ms / 1e6, 1) if traffic else None,
+                     "traffic_frac": round(traffic / kernel_ms / 1e6 / HBM_PEAK_GBS, 4) if traffic else None,
+                     "kernel": "k_dia_spmv<double,7,true>" if by_diagonals(sigma) else
                      f"k_csr5_tiles<double,{sigma},1,false,{'true' if codes else 'false'}>",
                      "kernel_ms": round(kernel_ms, 5),
                      "kernels_per_step": 1 if single_kernel else 2,
