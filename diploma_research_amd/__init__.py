@@ -5,8 +5,8 @@ Csr5.spmv, conjugate_gradient. Importing this package does not load the GPU
 library; the first call does (and fails loudly if it was not built).
 """
 from .csr5 import (Calibrator, CgResult, Coo, Csr, Csr5, Dimensions, SpmvData, conjugate_gradient,
-                   conjugate_gradient_multi)
+                   conjugate_gradient_multi, release_memory)
 from .native import DimError
 
 __all__ = ["Calibrator", "CgResult", "Coo", "Csr", "Csr5", "Dimensions", "SpmvData", "conjugate_gradient",
-           "conjugate_gradient_multi", "DimError"]
+           "conjugate_gradient_multi", "release_memory", "DimError"]

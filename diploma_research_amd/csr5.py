@@ -437,6 +437,12 @@ class CgResult:
     history: Optional[np.ndarray] = field(default=None, repr=False)
 
 
+def release_memory():
+    """Frees the device memory (at most 256 MiB on the current GPU) that the
+    library keeps of the last destroyed matrix for the next conversion."""
+    N.check(N.lib().dim_release_memory())
+
+
 def _cg_opts(rtol, max_iters, precision, check_every, refine_delta, hist, flags=0):
     prec = {"f64": N.DIM_CG_F64, "fp64": N.DIM_CG_F64, "f32-refined": N.DIM_CG_F32_REFINED,
             "fp32-ir": N.DIM_CG_F32_REFINED}[precision]

@@ -650,6 +650,11 @@ dim_status dim_csr5_destroy(dim_csr5* A) {
     return DIM_SUCCESS;
 }
 
+dim_status dim_release_memory(void) {
+    (void)drop_block();
+    return DIM_SUCCESS;
+}
+
 dim_status dim_csr5_get_info(const dim_csr5* A, dim_csr5_info* info) {
     if (dim_status st = check_handle(A))
         return st;

@@ -34,7 +34,8 @@ DIM_CG_NOALLOC_MAX_ROWS = 2097152
 # Every symbol include/dim_gpu.h declares (checked by the CPU test suite).
 EXPORTS = [
     "dim_last_error", "dim_status_string", "dim_version",
-    "dim_csr5_from_csr", "dim_csr5_from_csr_device", "dim_csr5_destroy", "dim_csr5_get_info",
+    "dim_csr5_from_csr", "dim_csr5_from_csr_device", "dim_csr5_destroy", "dim_release_memory",
+    "dim_csr5_get_info",
     "dim_csr5_copy_format", "dim_csr5_spmv", "dim_csr5_spmv_host", "dim_csr5_spmv_timed", "dim_csr5_block_rows", "dim_csr5_spmv_block", "dim_csr5_spmm",
     "dim_csr5_spmm_colmajor", "dim_csr5_spmv_transpose", "dim_csr5_sampled_outer", "dim_cg", "dim_cg_host", "dim_cg_noalloc",
     "dim_cg_multi", "dim_csr5_from_csr_batched",
@@ -91,6 +92,7 @@ def lib():
         "dim_csr5_from_csr": ([u32, u32, u64, vp, vp, vp, P(Csr5Opts), P(vp)], i32),
         "dim_csr5_from_csr_device": ([u32, u32, u64, vp, vp, vp, P(Csr5Opts), vp, P(vp)], i32),
         "dim_csr5_destroy": ([vp], i32),
+        "dim_release_memory": ([], i32),
         "dim_csr5_get_info": ([vp, P(Csr5Info)], i32),
         "dim_csr5_copy_format": ([vp, vp, vp, vp, vp, vp, P(u64), vp], i32),
         "dim_csr5_spmv": ([vp, i32, vp, u64, vp, u64, vp], i32),

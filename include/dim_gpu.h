@@ -96,6 +96,13 @@ dim_status dim_csr5_from_csr_device(uint32_t rows, uint32_t cols, uint64_t nnz, 
                                     void* stream, dim_csr5** out);
 
 dim_status dim_csr5_destroy(dim_csr5* A);
+
+/* Frees the device memory that the library keeps on the current device beyond
+ * its handles: one block of 16 to 256 MiB, the arrays of the last matrix
+ * destroyed, kept for the next conversion (the library gives it up by itself
+ * when the next one does not fit it or its own allocations find no room, but
+ * not for allocations of others). No reference counterpart. */
+dim_status dim_release_memory(void);
 dim_status dim_csr5_get_info(const dim_csr5* A, dim_csr5_info* info);
 
 /* Copies the format arrays to host buffers (any may be NULL): tile_ptr
