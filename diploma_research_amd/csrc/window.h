@@ -14,10 +14,20 @@ namespace dimgpu {
 constexpr uint32_t kWindowGroup = 16; // tiles whose column span is kept; wavefronts of a workgroup
 constexpr uint32_t kWindowMaxPer = 4;
 constexpr uint32_t kWindowMaxSigma = 16;
-// 64 workgroups: a smaller matrix would leave most CUs without one, and the tile
-// kernel spreads it over more. Just above the line (1054 tiles of 16 steps, band
-// of 14000 columns, FP64) the tile kernel takes 14.1 us, the windows 11.5.
+// 64 workgroups: the transposed and the FP32 products of smaller matrices leave
+// most CUs without one. In FP64 a workgroup has twice the bytes to move before
+// its first sum and needs more company: below 2048 tiles the tile kernel, which
+// spreads over more CUs, is faster (uneven rows of 12, sigma 16, microseconds,
+// tile kernel and windows: 1074 tiles, band 200: 10.8 and 15.0; 1097, band
+// 8000: 13.4 and 16.3; 2004, band 8000: 18.9 and 17.7; 2435, band 200: 19.0 and
+// 17.1). Narrow bands, whose x the tile kernel finds in L1 anyway, need 1.5M
+// elements besides (sigma 4, 2054 tiles, band 200: 5.7 and 6.9; sigma 8, 2924
+// tiles, band 200: 9.0 and 9.2); the others, with a window of half a
+// workgroup's elements or more, do not (sigma 4, 2514 tiles, band 2000: 8.5 and
+// 7.0).
 constexpr uint32_t kWindowMinTiles = 1024;
+constexpr uint32_t kWindowMinTiles64 = 2048;
+constexpr uint64_t kWindowNarrowElements = 1500000;
 
 // How a product is cut: workgroups of 16 wavefronts with `per` tiles each, and
 // the largest window, in entries of x; blocks == 0: the tile kernel's.
