@@ -235,10 +235,10 @@ void free_handle(dim_csr5* h);
 
 // The windows of a matrix on the device, from its spans on the host (window.h).
 inline void shape_windows(dim_csr5* h, const std::vector<uint32_t>& span, const std::vector<uint8_t>& tile_flags) {
-    h->win.f64 = window_shape(h->f.tiles, h->f.sigma, span, tile_flags, sizeof(double));
+    h->win.f64 = window_shape(h->f, span, tile_flags, sizeof(double));
     h->win.sums = window_sums_shape(h->f.tiles, h->f.sigma, span);
     if (h->f.vals32)
-        h->win.f32 = window_shape(h->f.tiles, h->f.sigma, span, tile_flags, sizeof(float));
+        h->win.f32 = window_shape(h->f, span, tile_flags, sizeof(float));
 }
 
 // New values (CSR order) into the tile layout, FP64 and, if kept, FP32, and into

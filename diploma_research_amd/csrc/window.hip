@@ -382,13 +382,17 @@ static WindowShape cut(uint32_t tiles, uint32_t sigma, const std::vector<uint32_
     return s;
 }
 
-WindowShape window_shape(uint32_t tiles, uint32_t sigma, const std::vector<uint32_t>& span,
+WindowShape window_shape(const DevFormat& A, const std::vector<uint32_t>& span,
                          const std::vector<uint8_t>& tile_flags, size_t vb) {
-    if (vb == sizeof(double) && tiles < kWindowMinTiles64)
+    const uint32_t tiles = A.tiles, sigma = A.sigma;
+    const bool f64 = vb == sizeof(double);
+    if (A.rows - A.n_empty > uint64_t{kWindowMaxStarts} * tiles || A.nnz < kWindowElements ||
+        (f64 && tiles < kWindowMinTiles64))
         return {};
     const WindowShape s = cut(tiles, sigma, span, (kLdsBytes - kStaticLds) / vb - kWaves * kStageRows - 2, 2);
-    const uint64_t each = uint64_t{kWindowGroup} * 64 * sigma * s.per; // elements of a workgroup
-    if (vb == sizeof(double) && 2 * uint64_t{s.width} < each && uint64_t{tiles} * 64 * sigma < kWindowNarrowElements)
+    const double each = double{kWindowGroup} * 64 * sigma * s.per; // elements of a workgroup
+    const double past = s.width - each * A.cols / A.nnz;
+    if (f64 && past < 0.4 * each && A.nnz < kWindowNarrowElements)
         return {};
     // every workgroup's first tile has a row start
     for (uint64_t t = 0; s.blocks && t < tiles; t += uint64_t{kWindowGroup} * s.per)

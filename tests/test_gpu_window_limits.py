@@ -20,7 +20,14 @@ def _lens(name, tiles, tile, rng):
     if name == "single elements":
         return np.ones(tiles * tile + 3, int)
     if name == "rows end with tiles":
-        return np.full(tiles * tile // 4, 4)
+        return np.full(tiles * tile // 8, 8)
+    if name == "runs of single elements":  # tiles with more row starts than a wavefront keeps sums
+        lens = np.full(tiles * tile // 15, 12)
+        for at in range(500, len(lens) - 3 * tile, len(lens) // 9):
+            lens[at: at + 2 * tile + 17] = 1
+        return lens
+    if name == "rows of three":
+        return rng.integers(1, 6, tiles * tile // 3)
     if name == "rows over wavefronts":
         lens = np.full((tiles // 8 + 1) * 6, tile)
         lens[3::6] = 4 * tile
@@ -32,8 +39,9 @@ def _lens(name, tiles, tile, rng):
 
 
 @pytest.mark.parametrize("name", ["uneven, some empty", "single elements", "rows end with tiles",
-                                  "rows over wavefronts", "rows over workgroups"])
-@pytest.mark.parametrize("sigma,tiles", [(4, 2040), (4, 2060), (4, 5870), (7, 2060), (8, 2930), (16, 2040), (16, 2060)])
+                                  "rows over wavefronts", "rows over workgroups", "runs of single elements",
+                                  "rows of three"])
+@pytest.mark.parametrize("sigma,tiles", [(4, 2060), (4, 2990), (4, 6500), (7, 2060), (8, 3500), (16, 2040), (16, 2400)])
 @pytest.mark.parametrize("band", [0, 6000])
 def test_products_on_both_sides_of_the_limits(cuda, name, sigma, tiles, band):
     """band 0: as narrow as the rows allow."""
