@@ -113,6 +113,7 @@ std::string build_batched(const std::vector<SystemCsr>& sys, uint32_t sigma, Hos
         if (dia) {
             out.dia_nd = std::max(out.dia_nd, f.dia_nd);
             out.dia_off.insert(out.dia_off.end(), f.dia_off.begin(), f.dia_off.end());
+            out.dia_meta.insert(out.dia_meta.end(), f.dia_meta.begin(), f.dia_meta.end());
         }
         rows += s.rows;
         tiles += f.tiles;
@@ -131,6 +132,7 @@ std::string build_batched(const std::vector<SystemCsr>& sys, uint32_t sigma, Hos
     if (!dia || uint64_t{rows} > (1u << 30)) {
         out.dia_nd = 0;
         out.dia_off.clear();
+        out.dia_meta.clear();
     }
     out.rows = out.cols = static_cast<uint32_t>(rows);
     out.tiles = static_cast<uint32_t>(tiles);
@@ -863,8 +865,10 @@ dim_status finish_batched(HostFormat& f, bool keep_f32, const std::vector<uint32
     // (only where the resident solver takes the batch)
     if (dia_nd && resident_batch(sys_row, f.dia_off, dia_nd).ok) {
         DiaForm D;
-        DIM_HIP_TRY(alloc_diagonals(h, dia_nd, 0, D));
+        DIM_HIP_TRY(alloc_diagonals(h, dia_nd, f.dia_meta.size(), D));
         if (D.nd) {
+            DIM_HIP_TRY(hipMemcpy(D.meta, f.dia_meta.data(), f.dia_meta.size() * sizeof(uint16_t),
+                                  hipMemcpyHostToDevice));
             int32_t* off = nullptr;
             DIM_HIP_TRY(upload(h, off, f.dia_off));
             D.sys_off = off;

@@ -23,7 +23,7 @@ struct DiaForm {
     const int32_t* sys_off = nullptr;
     double* v64 = nullptr;
     float* v32 = nullptr;
-    uint16_t* meta = nullptr; // (not kept for batches)
+    uint16_t* meta = nullptr;
     // plain products use it: the matrix keeps column codes or could, and no
     // row spans three lanes (the summation order is then the tile kernels')
     bool products = false;
