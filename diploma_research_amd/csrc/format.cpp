@@ -24,16 +24,22 @@ inline uint64_t upper_bound_idx(const uint32_t* a, uint64_t n, uint64_t v) {
     return static_cast<uint64_t>(std::upper_bound(a, a + n, v, [](uint64_t x, uint32_t y) { return x < y; }) - a) - 1;
 }
 
+// Rows (or lanes of elements) that are worth a thread.
+constexpr uint64_t kRangeRows = 2048;
+
+// f on ranges of [0, n), each of at least `least` (below that a range costs less
+// than the thread it would run on).
 template<typename F>
-void parallel_for(uint64_t n, F&& f) {
-    unsigned hw = std::max(1u, std::min(32u, std::thread::hardware_concurrency()));
-    if (n < 4096 || hw == 1) {
+void parallel_for(uint64_t n, F&& f, uint64_t least = 1) {
+    const uint64_t most = std::max<uint64_t>(1, std::min<uint64_t>(32, std::thread::hardware_concurrency()));
+    const uint64_t hw = std::min(most, n / least);
+    if (n < 4096 || hw <= 1) {
         f(uint64_t{0}, n);
         return;
     }
     std::vector<std::thread> th;
     uint64_t chunk = (n + hw - 1) / hw;
-    for (unsigned i = 0; i < hw; ++i) {
+    for (uint64_t i = 0; i < hw; ++i) {
         uint64_t b = i * chunk, e = std::min(n, b + chunk);
         if (b >= e)
             break;
@@ -43,38 +49,83 @@ void parallel_for(uint64_t n, F&& f) {
         t.join();
 }
 
-// The diagonals col - row of a matrix without empty rows, ascending; empty
-// when there are more than kMaxDiagonals, one lies beyond 32 bits, or x is
-// not below 4 GB (products of matrices kept by diagonals address x with
-// 32-bit byte offsets). Gathered per thread range and merged.
+// Whether the matrix may be kept by its diagonals col - row at all: no row is
+// empty and x is below 4 GB (products of matrices kept by diagonals address x
+// with 32-bit byte offsets).
+bool may_have_diagonals(const HostFormat& f) {
+    return !f.any_dirty && f.nnz && f.empty_rows.empty() && uint64_t{f.cols} * sizeof(double) <= (uint64_t{1} << 32);
+}
+
+// Adds the diagonals of rows [b, e) to d, until they are more than kMaxDiagonals.
+void add_diagonals(const uint32_t* row_ptr, const uint32_t* col_idx, uint64_t b, uint64_t e, std::vector<int64_t>& d) {
+    for (uint64_t r = b; r < e && d.size() <= kMaxDiagonals; ++r)
+        for (uint32_t k = row_ptr[r]; k < row_ptr[r + 1]; ++k) {
+            const int64_t v = int64_t{col_idx[k]} - static_cast<int64_t>(r);
+            if (std::find(d.begin(), d.end(), v) == d.end()) {
+                d.push_back(v);
+                if (d.size() > kMaxDiagonals)
+                    break;
+            }
+        }
+}
+
+// The diagonals of every row, ascending; empty when there are more than
+// kMaxDiagonals. Gathered per thread range and merged.
 std::vector<int64_t> find_diagonals(const HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx) {
-    if (f.any_dirty || !f.nnz || !f.empty_rows.empty() || uint64_t{f.cols} * sizeof(double) > (uint64_t{1} << 32))
-        return {};
     std::vector<int64_t> all;
     std::mutex m;
     bool too_many = false;
     parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
         std::vector<int64_t> d;
-        for (uint64_t r = b; r < e && d.size() <= kMaxDiagonals; ++r)
-            for (uint32_t k = row_ptr[r]; k < row_ptr[r + 1]; ++k) {
-                const int64_t v = int64_t{col_idx[k]} - static_cast<int64_t>(r);
-                if (std::find(d.begin(), d.end(), v) == d.end()) {
-                    d.push_back(v);
-                    if (d.size() > kMaxDiagonals)
-                        break;
-                }
-            }
+        add_diagonals(row_ptr, col_idx, b, e, d);
         std::lock_guard<std::mutex> g(m);
         if (d.size() > kMaxDiagonals)
             too_many = true;
         else
             all.insert(all.end(), d.begin(), d.end());
-    });
+    }, kRangeRows);
     std::sort(all.begin(), all.end());
     all.erase(std::unique(all.begin(), all.end()), all.end());
-    if (too_many || all.size() > kMaxDiagonals || all.front() < INT32_MIN || all.back() > INT32_MAX)
+    if (too_many || all.size() > kMaxDiagonals)
         return {};
     return all;
+}
+
+// Every row's word (HostFormat::dia_meta) from the diagonals `all`; false when
+// some row has an element on none of them, or its columns out of order, or one
+// twice.
+bool describe_rows(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx, const std::vector<int64_t>& all) {
+    f.dia_meta.resize(f.rows);
+    const uint32_t n = static_cast<uint32_t>(all.size());
+    std::atomic<bool> good{true};
+    const uint32_t sigma = f.sigma;
+    uint16_t* meta = f.dia_meta.data();
+    parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
+        uint32_t in = row_ptr[b] % sigma; // the row's first place in its lane
+        for (uint64_t r = b; r < e && good.load(std::memory_order_relaxed); ++r) {
+            const uint32_t e0 = row_ptr[r], len = row_ptr[r + 1] - e0;
+            const uint32_t left = len <= sigma ? sigma - in : len; // elements up to the lane's end
+            uint32_t held = 0, split = kDiaNoSplit, d = 0;
+            for (uint32_t k = 0; k < len; ++k) {
+                const int64_t v = int64_t{col_idx[e0 + k]} - static_cast<int64_t>(r);
+                while (d < n && all[d] != v)
+                    ++d;
+                if (d == n) {
+                    good.store(false, std::memory_order_relaxed);
+                    return;
+                }
+                held |= 1u << d;
+                split = k == left ? d : split;
+                ++d;
+            }
+            meta[r] = static_cast<uint16_t>(held | split << kDiaSplitShift);
+            for (in += len; in >= sigma;)
+                in -= sigma;
+        }
+    }, kRangeRows);
+    if (!good.load())
+        f.dia_meta.clear();
+    return good.load();
 }
 
 } // namespace
@@ -151,7 +202,7 @@ std::string build_format(uint32_t rows, uint32_t cols, uint64_t nnz, const uint3
             // another thread's rows except at range edges; use an atomic OR.
             __atomic_fetch_or(&f.bit_flag[t * kOmega + c], 1u << bit, __ATOMIC_RELAXED);
         }
-    });
+    }, kRangeRows);
 
     // tile flags and segment counts
     f.tile_flags.assign(T + 1, 0);
@@ -223,7 +274,25 @@ std::string build_format(uint32_t rows, uint32_t cols, uint64_t nnz, const uint3
     for (uint64_t r = 0; r < rows; ++r)
         if (row_ptr[r] == row_ptr[r + 1])
             f.empty_rows.push_back(static_cast<uint32_t>(r));
-    const std::vector<int64_t> diagonals = find_diagonals(f, row_ptr, col_idx);
+    // The diagonals of 64 rows are all of them in a stencil matrix, and already
+    // too many in most others: one pass then describes the rows, where finding
+    // the diagonals takes one of its own.
+    std::vector<int64_t> diagonals;
+    if (may_have_diagonals(f)) {
+        // (all over the matrix, by the golden ratio: a constant step may meet
+        // the same column of a grid again and again)
+        for (uint64_t i = 0; i < 64; ++i) {
+            const uint64_t r = ((i * 2654435769u + 0x80000000u) & 0xffffffffu) * rows >> 32;
+            add_diagonals(row_ptr, col_idx, r, r + 1, diagonals);
+        }
+        std::sort(diagonals.begin(), diagonals.end());
+        if (diagonals.size() > kMaxDiagonals)
+            diagonals.clear();
+        else if (diagonals.size() > kDiaMax || !describe_rows(f, row_ptr, col_idx, diagonals))
+            diagonals = find_diagonals(f, row_ptr, col_idx);
+    }
+    if (!diagonals.empty() && (diagonals.front() < INT32_MIN || diagonals.back() > INT32_MAX))
+        diagonals.clear();
     build_col_codes(f, row_ptr, col_idx, diagonals);
     build_diagonals(f, row_ptr, col_idx, diagonals);
     return {};
@@ -249,7 +318,7 @@ void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col
                 const int64_t v = int64_t{col_idx[k]} - static_cast<int64_t>(r);
                 code[k] = static_cast<uint8_t>(std::lower_bound(all.begin(), all.end(), v) - all.begin());
             }
-    });
+    }, kRangeRows);
     f.col_code.assign(uint64_t{f.tiles} * kOmega, 0);
     parallel_for(uint64_t{f.tiles} * kOmega, [&](uint64_t b, uint64_t e) {
         for (uint64_t w = b; w < e; ++w) {
@@ -259,45 +328,18 @@ void build_col_codes(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col
                 word |= uint32_t{code[first + r]} << (cb * r);
             f.col_code[w] = word;
         }
-    });
+    }, kRangeRows);
 }
 
 void build_diagonals(HostFormat& f, const uint32_t* row_ptr, const uint32_t* col_idx,
                      const std::vector<int64_t>& all) {
     f.dia_nd = 0;
     f.dia_off.clear();
-    f.dia_meta.clear();
     f.dia_rows_in_two_lanes = false;
-    // (rows plus an offset stay within 32 bits)
-    if (all.empty() || all.size() > kDiaMax || f.rows > (1u << 30))
-        return;
     const uint32_t nd = dia_kernel_diagonals(static_cast<uint32_t>(all.size()));
-    if (uint64_t{nd} * f.rows * 4 > f.nnz * 5)
-        return;
-    f.dia_meta.resize(f.rows);
-    std::atomic<bool> ordered{true};
-    parallel_for(f.rows, [&](uint64_t b, uint64_t e) {
-        for (uint64_t r = b; r < e; ++r) {
-            const uint32_t e0 = row_ptr[r], len = row_ptr[r + 1] - e0;
-            const uint32_t left = f.sigma - e0 % f.sigma; // elements up to the lane's end
-            uint32_t held = 0, split = kDiaNoSplit, d = 0;
-            for (uint32_t k = 0; k < len; ++k) {
-                const int64_t v = int64_t{col_idx[e0 + k]} - static_cast<int64_t>(r);
-                while (d < all.size() && all[d] != v)
-                    ++d;
-                if (d == all.size()) { // columns out of order, or one twice
-                    ordered.store(false, std::memory_order_relaxed);
-                    return;
-                }
-                held |= 1u << d;
-                if (k == left && len <= f.sigma)
-                    split = d;
-                ++d;
-            }
-            f.dia_meta[r] = static_cast<uint16_t>(held | split << kDiaSplitShift);
-        }
-    });
-    if (!ordered.load()) {
+    // (rows plus an offset stay within 32 bits)
+    if (all.empty() || all.size() > kDiaMax || f.rows > (1u << 30) || uint64_t{nd} * f.rows * 4 > f.nnz * 5 ||
+        (f.dia_meta.empty() && !describe_rows(f, row_ptr, col_idx, all))) {
         f.dia_meta.clear();
         return;
     }
