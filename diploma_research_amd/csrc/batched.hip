@@ -14,22 +14,23 @@
 // A batch of iterations is captured once in a hipGraph and replayed until
 // every system has stopped; the host looks at the state between batches.
 //
-// Batches whose systems are kept by diagonals and fit the chip iterate on
-// resident workgroups instead (resident.hip), with either flag; what follows
-// is for the rest.
+// Batches whose systems are kept by diagonals, fit an XCD each and are not too
+// many and small (plan_resident) iterate on resident workgroups instead
+// (resident.hip), with DIM_CG_PERSISTENT or without; what follows is for the
+// rest, and for when these workgroups cannot be seated.
 //
 // With DIM_CG_PERSISTENT the same three phases run inside one persistent
 // cooperative kernel that keeps the whole iteration loop on the device,
 // separated by grid barriers (see k_b_persistent); its iterates are bitwise
 // those of the launch sequence. Measured on the MI355X with 32 systems
-// (5.6M rows, 4792 iterations) it takes 0.81 s against 0.62 s: about 13 us
+// (5.6M rows, 4792 iterations) it takes 0.79 s against 0.59 s: about 13 us
 // more per grid barrier, three per iteration, than a kernel boundary inside
 // the graph, so the launch sequence stays the default.
 //
 // The adjoint solve with A^T products (DIM_CG_TRANSPOSE) uses the transposed
 // product and a separate p.q pass. Partial sums of a system are reduced in a
 // fixed order, so iterates are reproducible (apart from the transposed
-// product, which scatters with atomics).
+// product, whose sums have no fixed order).
 #include "handle.h"
 #include "resident.h"
 #include "spmv_impl.h"

@@ -119,8 +119,9 @@ __global__ __launch_bounds__(256) void k_dia_spmm_cols(DiaArgs a, int k, uint64_
 // divide k two lanes compute the same columns and write the same bits). A
 // wavefront so reads and writes consecutive memory, and a row's x entries for
 // all columns come with one line. The loads need no more than an element's
-// alignment. No transposes around it: 8 FP64 columns of 112^3 rows take 48 us
-// (261 MB at 5.4 TB/s), where the tile kernel between two transposes took 196.
+// alignment. No transposes around it: 8 FP64 columns of 112^3 rows, three
+// matrices and blocks in turn, take 71 us (61 where one stays in the Infinity
+// Cache), where the tile kernel between two transposes took 196.
 // One column per lane: 90 us, twice the loads.
 template<typename V, int ND, int W>
 __global__ __launch_bounds__(256) void k_dia_spmm_rows(DiaArgs a, uint32_t k, uint32_t L, uint32_t inv_L,
@@ -191,10 +192,13 @@ const V* values_of(const DiaForm& D) {
 // Infinity Cache, so that they do not push x out of L2 and two such matrices
 // in turn do not evict each other. 7 diagonals, FP64, 128^3 rows (155 MB): 26.5
 // us non-temporal, and with ordinary loads 20.1 us where one matrix is
-// multiplied over and over but 32.2 us for three in turn. FP32, 114^3 (56 MB):
-// 9.0-9.9 against 8.6 us, so smaller products use ordinary loads. Products of
-// several columns always do: their values are the smaller part, and 8 FP64
-// columns of 112^3 rows take 48 us so, 65 us non-temporal.
+// multiplied over and over but 32.2 us for three in turn: the line is drawn for
+// programs that touch other data between two products, and costs those that do
+// nothing else 6 us. FP32, 114^3 (56 MB): 9.0-9.9 against 8.6 us, so smaller
+// products use ordinary loads. Products of several columns always do: their
+// values are the smaller part. 8 FP64 columns, ordinary and non-temporal values:
+// 112^3 rows, three matrices in turn 73.4 and 72.1 us, one over and over 61.5 and
+// 66.5; 64^3 in turn 12.0 and 14.7; 160^3 in turn 207.6 and 205.1.
 template<typename V>
 bool stream_values(const DiaForm& D) {
     const uint64_t row = (uint64_t{D.nd} + 2) * sizeof(V) + sizeof(uint16_t);

@@ -46,7 +46,11 @@ struct ResidentState {
 
 constexpr uint32_t kResidentXcds = 8;
 constexpr uint32_t kResidentCus = 32; // workgroups (one per CU) of an XCD
-constexpr uint32_t kResidentRows = 1u << 21; // the largest system: 8192 rows per CU
+// The largest system: 8192 rows per CU of the whole chip, and only as the one
+// job of a solve. Several jobs have an XCD each at most, with the values in
+// registers: 131072 rows (FP64, 5 or 7 diagonals; 3: 262144, 9: 65536; FP32:
+// 262144, 9 diagonals 131072), or the launch sequence takes them all.
+constexpr uint32_t kResidentRows = 1u << 21;
 
 // How long a solve waits for the chip, first for another solve of the process
 // and then for its own workgroups to be running (CUs held by other streams or

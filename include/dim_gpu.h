@@ -14,7 +14,13 @@
  *   - a dim_csr5 handle owns its device arrays and a small scratch area (the
  *     counterpart of the reference's calibrator, csr5/calibrator.h:14-31), so
  *     calls on ONE handle must not overlap (same rule as the reference's
- *     shared calibrator); different handles are independent.
+ *     shared calibrator); different handles are independent, but for the
+ *     chip: a CG solve whose system is kept by diagonals (a stencil matrix)
+ *     takes every CU at once while it starts and, where it is large, for its
+ *     whole iteration. Such solves of one process run one after another; one
+ *     that would wait more than 10 ms for another solve or for CUs that other
+ *     work holds iterates by a sequence of launches instead, with the same
+ *     stop test and other rounding.
  *   - y = A*x OVERWRITES y, including 0 in empty rows (the reference adds into
  *     a zero-filled y and skips empty rows, csr5.h:526-538, 750-754).
  */
@@ -166,8 +172,10 @@ dim_status dim_csr5_spmm(const dim_csr5* A, dim_dtype dtype, uint32_t k, const v
 dim_status dim_csr5_spmm_colmajor(const dim_csr5* A, dim_dtype dtype, uint32_t k, const void* X, uint64_t ldx,
                                   void* Y, uint64_t ldy, void* stream);
 
-/* y = A^T x (x: rows entries, y: cols entries). No reference counterpart;
- * used by the adjoint. */
+/* y = A^T x (x: rows entries, y: cols entries). The first product of a matrix
+ * of 32768 elements or more, outside a capture, makes a plan that the handle
+ * keeps: 10 bytes per element, or the sums of LDS windows for matrices within
+ * a band. No reference counterpart; used by the adjoint. */
 dim_status dim_csr5_spmv_transpose(const dim_csr5* A, dim_dtype dtype, const void* x, void* y, void* stream);
 
 /* out[e] = scale * u[row(e)] * v[col(e)] for every stored element, in the
@@ -187,7 +195,8 @@ typedef struct dim_cg_opts {
     double rtol;           /* stop when ||r|| / ||b|| <= rtol */
     uint32_t max_iters;    /* iteration cap (for F32_REFINED: inner iterations in total) */
     uint32_t precision;    /* dim_cg_precision */
-    uint32_t check_every;  /* iterations between host convergence checks (0 = 16) */
+    uint32_t check_every;  /* iterations between host convergence checks (0 = 16); solves by resident
+                              workgroups test after every iteration on the device instead */
     double refine_delta;   /* F32_REFINED: FP64 residual replacement when ||r|| drops by this factor (0 = 0.1) */
     double* history;       /* optional HOST array of max_iters+1: ||r_i||/||b|| (recursive residual) */
     uint32_t flags;        /* DIM_CG_* below; batched only */
@@ -196,7 +205,10 @@ typedef struct dim_cg_opts {
 #define DIM_CG_TRANSPOSE 1u
 /* run the whole iteration loop in one persistent cooperative kernel with
  * grid barriers instead of replaying a captured launch sequence (not with
- * DIM_CG_TRANSPOSE; DIM_UNSUPPORTED when the kernel cannot be resident) */
+ * DIM_CG_TRANSPOSE; DIM_UNSUPPORTED when the kernel cannot be resident).
+ * Batches whose systems are kept by diagonals and fit the chip iterate on
+ * resident workgroups with or without the flag, which then only says what
+ * takes their place when these cannot be seated. */
 #define DIM_CG_PERSISTENT 2u
 
 typedef struct dim_cg_result {
@@ -237,7 +249,8 @@ dim_status dim_cg_host(const dim_csr5* A, const double* b, double* x, const dim_
  * opts->history NULL, the matrix on the current device. Calls that overlap
  * on one GPU (other threads or streams) race on the array: serialise them.
  * res->seconds is the host wall time of the call. Results equal dim_cg's
- * bit for bit (same kernels in the same order). */
+ * bit for bit (same kernels in the same order) unless other work on the GPU
+ * makes one of the two iterate by launches. */
 #define DIM_CG_NOALLOC_MAX_ROWS 2097152u
 #define DIM_CG_NOALLOC_BYTES (1024u + 4u * 256u * 16u * 8u + 24u * DIM_CG_NOALLOC_MAX_ROWS + 8u * 256u)
 dim_status dim_cg_noalloc(const dim_csr5* A, const double* b, double* x, const dim_cg_opts* opts,
@@ -252,9 +265,12 @@ dim_status dim_cg_multi(const dim_csr5* A, uint32_t k, const double* B, double* 
  * block-diagonal matrix built with dim_csr5_from_csr_batched (host CSR arrays
  * per system, each square; rows[i] rows and nnz[i] entries), B/X hold the
  * systems' vectors back to back (DEVICE, FP64). Every system keeps its own
- * step lengths and stop test; a batch of iterations is captured once in a
- * hipGraph and replayed until every system has stopped. res has n_systems
- * entries. With opts->flags & DIM_CG_TRANSPOSE the products use A^T (the
+ * step lengths and stop test. Systems kept by diagonals of at most
+ * 131,072 rows each (3 diagonals: 262,144, 9: 65,536) iterate on resident
+ * workgroups, unless they are so many and small that the launch sequence,
+ * which takes them side by side, is faster; otherwise a batch of iterations is
+ * captured once in a hipGraph and replayed until every system has stopped.
+ * res has n_systems entries. With opts->flags & DIM_CG_TRANSPOSE the products use A^T (the
  * adjoint solve). No reference counterpart (the reference solves one system
  * per process). Padding elements of each system's last tile are stored as
  * 0 * x[first row of the system], so x must be finite. The batch handle keeps
