@@ -14,8 +14,10 @@ namespace dimgpu {
 constexpr uint32_t kWindowGroup = 16; // tiles whose column span is kept; wavefronts of a workgroup
 constexpr uint32_t kWindowMaxPer = 4;
 constexpr uint32_t kWindowMaxSigma = 16;
-// 64 workgroups: the transposed products of smaller matrices leave most CUs
-// without one.
+// 64 workgroups: smaller matrices leave most CUs without one. Not the crossing
+// but a little above it: FP32 products at 1074 tiles of sigma 16 take 9.5 us by
+// the tile kernel and 9.2 by windows, transposed ones 19.5 sorted at 940 tiles
+// and 15.2 by windows at 1031 (band of 2000).
 constexpr uint32_t kWindowMinTiles = 1024;
 
 // What else a plain product by windows needs to be the faster one; uneven rows,

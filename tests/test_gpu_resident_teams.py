@@ -198,6 +198,8 @@ def test_solves_of_other_handles_are_not_held_up(cuda):
     conjugate_gradient(long, b, rtol=1e-1, max_iters=5)
     s_long, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(8)]
     bd, marks = to_dev(bs), [torch.zeros(8, device="cuda") for _ in others]
+    for mark in marks:  # (loads the kernel)
+        mark.add_(1)
     torch.cuda.synchronize()
     ended = {}
 
@@ -210,14 +212,16 @@ def test_solves_of_other_handles_are_not_held_up(cuda):
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     t.start()
+    time.sleep(0.05)  # (the long solve is on the GPU by then)
     # a stream that does not share the long solve's hardware queue
     events = [torch.cuda.Event() for _ in others]
     for q, e, mark in zip(others, events, marks):
         with torch.cuda.stream(q):
             mark.add_(1)
         e.record(q)
-    time.sleep(0.05)
-    free = [q for q, e in zip(others, events) if e.query()]
+    free = []
+    while not free and t.is_alive():
+        free = [q for q, e in zip(others, events) if e.query()]
     assert free and t.is_alive()
     x, r = conjugate_gradient(short, bd, x=x0, rtol=1e-10, stream=free[0])
     ended["short"] = time.perf_counter()
