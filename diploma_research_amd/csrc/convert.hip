@@ -114,7 +114,7 @@ template<typename W>
 __global__ __launch_bounds__(kT) void k_tiles(uint32_t T, uint32_t rows, uint32_t nnz, uint32_t sigma,
                                               const uint32_t* __restrict__ rp, uint32_t* __restrict__ tile_ptr,
                                               W* __restrict__ bits, uint8_t* __restrict__ tile_flags,
-                                              uint32_t* __restrict__ nseg_dirty, Counts* counts) {
+                                              uint32_t* __restrict__ nseg_dirty) {
     __shared__ uint32_t words[kT / 64][64];
     const uint32_t t = blockIdx.x * (kT / 64) + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -157,21 +157,22 @@ __global__ __launch_bounds__(kT) void k_tiles(uint32_t T, uint32_t rows, uint32_
         tile_ptr[t] = start | (dirty ? kDirty : 0u);
         tile_flags[t] = static_cast<uint8_t>(((word & 1u) ? kStartsRow : 0) | (n > 1 ? kMultiSeg : 0));
         nseg_dirty[t] = dirty ? static_cast<uint32_t>(n) : 0u;
-        if (dirty)
-            atomicAdd(&counts->n_dirty, 1u);
     }
 }
 
-// Exclusive scan of in[0..n) to out[0..n], out[n] the total (also to *total), by
-// one workgroup.
+// Exclusive scan of in[0..n) to out[0..n], out[n] the total (also to *total; the
+// number of entries that are not 0 is added to *nonzero), by one workgroup.
+// (Dirty tiles are counted here: an atomic add of each, 586k of them in 150M
+// elements at sigma 4, made a conversion of 3.2 ms take 8.7.)
 __global__ __launch_bounds__(1024) void k_scan(uint32_t n, const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                               uint32_t* total) {
+                                               uint32_t* total, uint32_t* nonzero) {
     __shared__ uint32_t wave_sum[16], carry_s;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t carry = 0;
+    uint32_t carry = 0, filled = 0;
     for (uint32_t i0 = 0; i0 < n; i0 += 1024) {
         const uint32_t i = i0 + threadIdx.x;
         const uint32_t v = i < n ? in[i] : 0u;
+        filled += v ? 1u : 0u;
         const uint32_t incl = static_cast<uint32_t>(wave_incl_scan(static_cast<int>(v), lane));
         if (lane == 63)
             wave_sum[w] = incl;
@@ -191,6 +192,8 @@ __global__ __launch_bounds__(1024) void k_scan(uint32_t n, const uint32_t* __res
         if (total)
             *total = carry;
     }
+    if (nonzero && filled)
+        atomicAdd(nonzero, filled);
 }
 
 // Segment -> row offsets of dirty tiles: segment 0 lies in the tile's first row,
@@ -402,7 +405,7 @@ dim_status convert(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t* r
                        n_empty == 0, d.tile_ptr, d.tile_flags, d.tile_desc_offset_ptr, d.tile_desc_offset, h->s.queue, h->win.span);
     if (T) {
         hipLaunchKernelGGL((k_tiles<W>), tile_grid, block, 0, s, T, rows, n32, sigma, rp, d.tile_ptr, bits,
-                           d.tile_flags, nseg_dirty, counts);
+                           d.tile_flags, nseg_dirty);
         switch (sigma) {
 #define DIM_TRANSPOSE(S)                                                                                              \
     case S:                                                                                                           \
@@ -416,14 +419,14 @@ dim_status convert(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t* r
     }
     if (n_empty) {
         hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, T, static_cast<const uint32_t*>(nseg_dirty),
-                           d.tile_desc_offset_ptr, &counts->ntdo);
+                           d.tile_desc_offset_ptr, &counts->ntdo, &counts->n_dirty);
         if (T)
             hipLaunchKernelGGL(k_tile_offsets, tile_grid, block, 0, s, T, rows, n32, static_cast<uint32_t>(tile), rp,
                                static_cast<const uint32_t*>(d.tile_ptr),
                                static_cast<const uint32_t*>(d.tile_desc_offset_ptr), d.tile_desc_offset);
         hipLaunchKernelGGL(k_count_empty, dim3(row_blocks), block, 0, s, rows, rp, empty_counts);
         hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, row_blocks, static_cast<const uint32_t*>(empty_counts),
-                           empty_first, static_cast<uint32_t*>(nullptr));
+                           empty_first, static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr));
         hipLaunchKernelGGL(k_list_empty, dim3(row_blocks), dim3(64), 0, s, rows, rp,
                            static_cast<const uint32_t*>(empty_first), d.empty_rows);
         DIM_HIP_TRY(hipMemcpyAsync(&got, counts, sizeof(Counts), hipMemcpyDeviceToHost, s));
